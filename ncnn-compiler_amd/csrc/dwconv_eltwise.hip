@@ -645,6 +645,9 @@ static int dw_bands(int planes, int oh, int ow, int kh, int kw, int sh, int dh, 
 
 int launch_dwconv_int8(const nhip_conv_plan* p, const void* in, int in_is_i8, void* out, int n, int h, int w,
                        int oh, int ow, hipStream_t s) {
+  // 3x3 and 5x5 at stride 1 or 2 without dilation (dw_int8.hip); the kernel
+  // below takes the other windows and rows too wide to stage
+  if (dw_int8_runs_supported(p, n, h, w, oh)) return launch_dw_int8_runs(p, in, in_is_i8, out, n, h, w, oh, ow, s);
   DwI8Args a{};
   a.x = in;
   a.y = out;

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include <string>
+#include <vector>
 
 #include "../../include/nhip.h"
 
@@ -198,6 +199,9 @@ struct nhip_conv_plan {
   // wave's load of a k step is 1 KB contiguous.  Only when that kernel can
   // take the plan (kred_pad == kRwKred, m_pad a multiple of 128).
   int8_t* weight_i8_frag = nullptr;
+  // int8 depthwise plans of dw_int8.hip: [C][K][ceil(K/4)] words, a row's taps
+  // as bytes, zero padded.
+  int32_t* weight_dw_pack = nullptr;
   float* recip = nullptr;
   float input_scale = 1.0f, output_scale = 1.0f;
   int32_t scale_term = 0;
@@ -275,6 +279,12 @@ int launch_dwconv_f32(const nhip_conv_plan* p, const float* in, float* out,
 int launch_dwconv_int8(const nhip_conv_plan* p, const void* in, int in_is_i8,
                        void* out, int n, int h, int w, int oh, int ow,
                        hipStream_t s);
+// dw_int8.hip: int8 depthwise 3x3 and 5x5, stride 1 or 2, 4 x 4 outputs per
+// thread on dot4.
+std::vector<int32_t> dw_int8_pack(const nhip_conv_plan* p, const int8_t* wq);
+bool dw_int8_runs_supported(const nhip_conv_plan* p, int n, int h, int w, int oh);
+int launch_dw_int8_runs(const nhip_conv_plan* p, const void* in, int in_is_i8, void* out, int n, int h, int w, int oh,
+                        int ow, hipStream_t s);
 int launch_innerproduct_f32(const nhip_ip_plan* p, const float* in,
                             float* out, int m, void* ws, uint64_t ws_bytes,
                             hipStream_t s);

@@ -355,6 +355,7 @@ void free_plan(nhip_conv_plan* p) {
   (void)hipFree(p->ktab);
   (void)hipFree(p->weight_i8);
   (void)hipFree(p->weight_i8_frag);
+  (void)hipFree(p->weight_dw_pack);
   (void)hipFree(p->recip);
   delete p;
 }
@@ -898,6 +899,9 @@ int nhip_dwconv2d_int8_create(const nhip_conv_desc* d, const void* weight, int32
     rc[c] = ws == 0.0f ? 0.0f : r;
   }
   int st = upload(&p->weight_i8, wq, "hipMalloc(dw int8 weight)");
+  const std::vector<int32_t> packed = dw_int8_pack(p, wq.data());
+  if (st == NHIP_STATUS_SUCCESS && !packed.empty())
+    st = upload(&p->weight_dw_pack, packed, "hipMalloc(dw int8 weight, words)");
   if (st == NHIP_STATUS_SUCCESS) st = upload(&p->recip, rc, "hipMalloc(dw int8 reciprocal)");
   if (st == NHIP_STATUS_SUCCESS) st = upload_bias(p, d->bias_term ? bias : nullptr, C, C);
   if (st != NHIP_STATUS_SUCCESS) {
