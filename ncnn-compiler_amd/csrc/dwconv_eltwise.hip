@@ -599,6 +599,117 @@ __global__ void dequantize_kernel(const int32_t* x, float* y, int64_t n, int c, 
   }
 }
 
+// The three kernels above on groups of four elements, for fewer than 2^31 of
+// them: a 16-byte load, one 4-byte (int8) or 16-byte (fp32) store, four groups
+// per thread 4 KB apart in flight as in eltwise_v4_kernel.  They are bound by
+// HBM; what the element loops lose it to is a 64-bit division and up to three
+// parameter loads per element, and a one-byte store per lane.  A wave's 64
+// groups are 256 consecutive elements, so from planes of 256 elements on (MODE
+// 2) they belong to at most two channels: both channels' parameters are
+// wave-uniform, requested together with the data, and each element picks one.
+// Smaller planes (MODE 1) find each group's channel, and the next one where a
+// plane ends inside it, per lane; planes of fewer than four elements per
+// element.  MODE 0: one entry for all channels.  32 x 144 x 56 x 56 int32 ->
+// int8 per channel: 35 -> 16.2 us (72 MB, 4.5 TB/s); per-lane parameters for
+// such planes took 55 us, the parameter loads outnumbering the data's.
+// Buffers need only the alignment of their elements.
+// OP 0 quantize, 1 requantize, 2 dequantize.
+struct QuantArgs {
+  int64_t n;                // elements
+  int plane, c;
+  FastDiv plane_div, c_div;
+  int isn, osn, bn;         // entries of the scales and the bias: 1 or c (bias: 0 none)
+  int act;
+};
+struct QuantCh {
+  float is, os, b;
+};
+
+template <int OP, int MODE>
+__global__ __launch_bounds__(256) void quant_v4_kernel(const int* __restrict__ x, void* __restrict__ y,
+                                                       const float* __restrict__ isc, const float* __restrict__ osc,
+                                                       const float* __restrict__ bias, QuantArgs a) {
+  constexpr int kPer = 4;
+  auto channel = [&](int ch) {
+    QuantCh r{0.f, 0.f, 0.f};
+    if (OP != 0) r.is = isc[a.isn == 1 ? 0 : ch];
+    if (OP != 2) r.os = osc[a.osn == 1 ? 0 : ch];
+    if (OP != 0 && a.bn != 0) r.b = bias[a.bn == 1 ? 0 : ch];
+    return r;
+  };
+  auto channel_of = [&](int plane) { return plane - fdiv(plane, a.c_div) * a.c; };
+  auto value = [&](int raw, const QuantCh& p) {
+#pragma clang fp contract(off)
+    if (OP == 0) return __int_as_float(raw);
+    float f = (float)raw * p.is;
+    if (a.bn != 0) f = f + p.b;
+    if (OP == 1 && a.act == NHIP_ACT_RELU) f = f < 0.f ? 0.f : f;
+    return f;
+  };
+  const int64_t n4 = a.n >> 2, chunk = (int64_t)kPer * blockDim.x;
+  const int lane = threadIdx.x & 63;
+  const QuantCh only = MODE == 0 ? channel(0) : QuantCh{};
+  for (int64_t base = (int64_t)blockIdx.x * chunk; base < n4; base += (int64_t)gridDim.x * chunk) {
+    v4i v[kPer];
+    QuantCh p0[kPer], p1[kPer];
+    int left[kPer];  // elements of the first channel, from the wave's (MODE 2) or the lane's (MODE 1) first on
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int64_t i = base + u * blockDim.x + threadIdx.x;
+      if (i < n4) __builtin_memcpy(&v[u], x + 4 * i, 16);
+      if (MODE == 0) continue;
+      const int64_t first = MODE == 2 ? i - lane : i;
+      int e0 = (int)min(4 * first, a.n - 1);
+      if (MODE == 2) e0 = __builtin_amdgcn_readfirstlane(e0);
+      const int pl = fdiv(e0, a.plane_div), ch = channel_of(pl);
+      left[u] = a.plane - (e0 - pl * a.plane);
+      p0[u] = channel(ch);
+      p1[u] = channel(ch + 1 == a.c ? 0 : ch + 1);
+    }
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      const int64_t i = base + u * blockDim.x + threadIdx.x;
+      if (i >= n4) continue;
+      QuantCh p[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (MODE == 0)
+          p[e] = only;
+        else
+          p[e] = (MODE == 2 ? 4 * lane + e : e) < left[u] ? p0[u] : p1[u];
+      }
+      if (MODE == 1 && a.plane < 4) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[e] = channel(channel_of(fdiv((int)(4 * i) + e, a.plane_div)));
+      }
+      float f[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int raw = v[u][e];
+        f[e] = value(raw, p[e]);
+      }
+      if constexpr (OP == 2) {
+        const v4f o{f[0], f[1], f[2], f[3]};
+        __builtin_memcpy(static_cast<float*>(y) + 4 * i, &o, 16);
+      } else {
+        const uint32_t o = pack_i8x4(quantize_q(f[0], p[0].os), quantize_q(f[1], p[1].os), quantize_q(f[2], p[2].os),
+                                     quantize_q(f[3], p[3].os));
+        __builtin_memcpy(static_cast<int8_t*>(y) + 4 * i, &o, 4);
+      }
+    }
+  }
+  // the last n % 4 elements
+  if (blockIdx.x == 0 && (int)threadIdx.x < (int)(a.n & 3)) {
+    const int e = (int)(4 * n4) + (int)threadIdx.x;
+    const QuantCh p = MODE == 0 ? only : channel(channel_of(fdiv(e, a.plane_div)));
+    const float f = value(x[e], p);
+    if constexpr (OP == 2)
+      static_cast<float*>(y)[e] = f;
+    else
+      static_cast<int8_t*>(y)[e] = quantize_i8(f, p.os);
+  }
+}
+
 unsigned grid_for(int64_t n) {
   const int64_t blocks = ceil_div(n, 256);
   const int64_t cap = 64LL * cu_count();
@@ -611,6 +722,34 @@ unsigned grid_v4(int64_t n4) {
   const int64_t blocks = ceil_div(n4, 4 * 256);
   const int64_t cap = 16LL * cu_count();
   return (unsigned)(blocks < cap ? (blocks > 0 ? blocks : 1) : cap);
+}
+
+// The vector kernels' launch for fewer than 2^31 elements; the element loops
+// take the rest.
+bool quant_v4_selected(int64_t count) { return count < (int64_t(1) << 31); }
+
+template <int OP>
+int launch_quant_v4(const char* name, const void* x, void* y, const float* isc, int isn, const float* osc, int osn,
+                    const float* bias, int bn, int act, int64_t count, int64_t plane, int c, hipStream_t s) {
+  QuantArgs a{};
+  a.n = count;
+  a.plane = (int)plane;
+  a.c = c;
+  a.plane_div = fast_div((uint32_t)plane);
+  a.c_div = fast_div((uint32_t)c);
+  a.isn = isn;
+  a.osn = osn;
+  a.bn = bias ? bn : 0;
+  a.act = act;
+  const dim3 grid(grid_v4(std::max<int64_t>(1, count / 4)));
+  const int* xi = static_cast<const int*>(x);
+  if (isn <= 1 && osn <= 1 && a.bn <= 1)
+    NHIP_LAUNCH(name, (quant_v4_kernel<OP, 0>), grid, dim3(256), 0, s, xi, y, isc, osc, bias, a);
+  else if (plane >= 256)
+    NHIP_LAUNCH(name, (quant_v4_kernel<OP, 2>), grid, dim3(256), 0, s, xi, y, isc, osc, bias, a);
+  else
+    NHIP_LAUNCH(name, (quant_v4_kernel<OP, 1>), grid, dim3(256), 0, s, xi, y, isc, osc, bias, a);
+  return check_launch(name);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -858,6 +997,9 @@ int nhip_quantize_f32_i8(const float* input, int8_t* output, int32_t n, int32_t 
     return fail(NHIP_STATUS_INVALID_SHAPE, "quantize: invalid shape or scale count");
   const int64_t count = (int64_t)n * c * plane;
   if (count == 0) return ok();
+  if (quant_v4_selected(count))
+    return launch_quant_v4<0>("quantize_f32_i8", input, output, nullptr, 0, scale, scale_count, nullptr, 0, 0, count, plane, c,
+                               as_stream(stream));
   NHIP_LAUNCH("quantize_f32_i8", quantize_f32_i8_kernel, dim3(grid_for(count)), dim3(256), 0, as_stream(stream),
                      input, output, count, c, plane, scale, scale_count);
   return check_launch("quantize_f32_i8");
@@ -875,6 +1017,10 @@ int nhip_requantize_i32_i8(const int32_t* input, int8_t* output, int32_t n, int3
     return fail(NHIP_STATUS_INVALID_SHAPE, "requantize: invalid shape or scale count");
   const int64_t count = (int64_t)n * c * plane;
   if (count == 0) return ok();
+  if (quant_v4_selected(count))
+    return launch_quant_v4<1>("requantize_i32_i8", input, output, in_scale, in_scale_count, out_scale, out_scale_count, bias,
+                               bias_count, activation, count, plane, c,
+                               as_stream(stream));
   NHIP_LAUNCH("requantize_i32_i8", requantize_kernel, dim3(grid_for(count)), dim3(256), 0, as_stream(stream),
                      input, output, count, c, plane, in_scale, in_scale_count, out_scale,
                      out_scale_count, bias, bias_count, activation);
@@ -890,6 +1036,9 @@ int nhip_dequantize_i32_f32(const int32_t* input, float* output, int32_t n, int3
     return fail(NHIP_STATUS_INVALID_SHAPE, "dequantize: invalid shape or scale count");
   const int64_t count = (int64_t)n * c * plane;
   if (count == 0) return ok();
+  if (quant_v4_selected(count))
+    return launch_quant_v4<2>("dequantize_i32_f32", input, output, scale, scale_count, nullptr, 0, bias, bias_count, 0, count, plane, c,
+                               as_stream(stream));
   NHIP_LAUNCH("dequantize_i32_f32", dequantize_kernel, dim3(grid_for(count)), dim3(256), 0, as_stream(stream),
                      input, output, count, c, plane, scale, scale_count, bias, bias_count);
   return check_launch("dequantize_i32_f32");
