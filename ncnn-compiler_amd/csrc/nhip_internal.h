@@ -200,7 +200,7 @@ struct nhip_conv_plan {
   // take the plan (kred_pad == kRwKred, m_pad a multiple of 128).
   int8_t* weight_i8_frag = nullptr;
   // int8 depthwise plans of dw_int8.hip: [C][K][ceil(K/4)] words, a row's taps
-  // as bytes, zero padded.
+  // as bytes, zero padded; inside weight_i8's buffer, after the bytes.
   int32_t* weight_dw_pack = nullptr;
   float* recip = nullptr;
   float input_scale = 1.0f, output_scale = 1.0f;

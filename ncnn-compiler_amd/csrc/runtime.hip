@@ -355,7 +355,6 @@ void free_plan(nhip_conv_plan* p) {
   (void)hipFree(p->ktab);
   (void)hipFree(p->weight_i8);
   (void)hipFree(p->weight_i8_frag);
-  (void)hipFree(p->weight_dw_pack);
   (void)hipFree(p->recip);
   delete p;
 }
@@ -898,10 +897,16 @@ int nhip_dwconv2d_int8_create(const nhip_conv_desc* d, const void* weight, int32
     const float r = 1.0f / combined;
     rc[c] = ws == 0.0f ? 0.0f : r;
   }
-  int st = upload(&p->weight_i8, wq, "hipMalloc(dw int8 weight)");
+  // the word copy follows the bytes in the same buffer (one upload)
   const std::vector<int32_t> packed = dw_int8_pack(p, wq.data());
+  const size_t pack_at = (size_t)round_up((int64_t)wq.size(), 16);
+  if (!packed.empty()) {
+    wq.resize(pack_at + packed.size() * 4, 0);
+    std::memcpy(wq.data() + pack_at, packed.data(), packed.size() * 4);
+  }
+  int st = upload(&p->weight_i8, wq, "hipMalloc(dw int8 weight)");
   if (st == NHIP_STATUS_SUCCESS && !packed.empty())
-    st = upload(&p->weight_dw_pack, packed, "hipMalloc(dw int8 weight, words)");
+    p->weight_dw_pack = reinterpret_cast<int32_t*>(p->weight_i8 + pack_at);
   if (st == NHIP_STATUS_SUCCESS) st = upload(&p->recip, rc, "hipMalloc(dw int8 reciprocal)");
   if (st == NHIP_STATUS_SUCCESS) st = upload_bias(p, d->bias_term ? bias : nullptr, C, C);
   if (st != NHIP_STATUS_SUCCESS) {
