@@ -203,9 +203,13 @@ def _torch_dtype(np_dtype):
 
 
 def _stream(stream=None):
-    torch = _torch()
-    s = torch.cuda.current_stream() if stream is None else stream
-    return _P(s.cuda_stream)
+    """The given stream's handle, or the current device's current stream's
+    (its handle alone: building torch's Stream object took 3 of a call's 8
+    us)."""
+    if stream is not None:
+        return _P(stream.cuda_stream)
+    C = _torch()._C
+    return _P(C._cuda_getCurrentRawStream(C._cuda_getDevice()))
 
 
 def _dev(t, dtype):
@@ -294,8 +298,8 @@ class Conv2dF32(_Plan):
         torch = _torch()
         x = _dev(x, torch.float32)
         n, c, h, w = x.shape
-        oh, ow = output_shape(self.desc, h, w)
         if out is None:
+            oh, ow = output_shape(self.desc, h, w)
             out = torch.empty((n, self.desc.num_output, oh, ow), dtype=torch.float32, device=x.device)
         if residual is not None:
             residual = _dev(residual, torch.float32)
@@ -334,9 +338,9 @@ class Conv2dInt8(_Plan):
             raise TypeError("int8 conv input must be a float32 or int8 device tensor")
         x = x.contiguous()
         n, c, h, w = x.shape
-        oh, ow = output_shape(self.desc, h, w)
-        odt = torch.int8 if self.desc.int8_scale_term > 100 else torch.float32
         if out is None:
+            oh, ow = output_shape(self.desc, h, w)
+            odt = torch.int8 if self.desc.int8_scale_term > 100 else torch.float32
             out = torch.empty((n, self.desc.num_output, oh, ow), dtype=odt, device=x.device)
         if workspace is None:
             workspace, nbytes = _workspace(self.workspace_size(n, h, w), x.device)
@@ -363,8 +367,8 @@ class DwConv2dF32(_Plan):
         torch = _torch()
         x = _dev(x, torch.float32)
         n, c, h, w = x.shape
-        oh, ow = output_shape(self.desc, h, w)
         if out is None:
+            oh, ow = output_shape(self.desc, h, w)
             out = torch.empty((n, self.desc.num_output, oh, ow), dtype=torch.float32, device=x.device)
         check(load().nhip_dwconv2d_f32_forward(self.handle, _ptr(x), _ptr(out), n, h, w, _stream(stream)))
         return out
@@ -435,9 +439,9 @@ class DwConv2dInt8(_Plan):
             raise TypeError("int8 depthwise input must be a float32 or int8 device tensor")
         x = x.contiguous()
         n, c, h, w = x.shape
-        oh, ow = output_shape(self.desc, h, w)
-        odt = torch.int8 if self.desc.int8_scale_term > 100 else torch.float32
         if out is None:
+            oh, ow = output_shape(self.desc, h, w)
+            odt = torch.int8 if self.desc.int8_scale_term > 100 else torch.float32
             out = torch.empty((n, c, oh, ow), dtype=odt, device=x.device)
         check(load().nhip_dwconv2d_int8_forward(self.handle, _ptr(x), 1 if x.dtype == torch.int8 else 0, _ptr(out),
                                                 n, h, w, _stream(stream)))
@@ -569,13 +573,35 @@ def global_avgpool(x, stream=None):
     return out
 
 
+def _params(device, stream, *values):
+    """fp32 device arrays of per-channel (or single) parameters; None stays
+    None.  On the current stream they go up in one asynchronous copy from
+    pinned memory (torch's host allocator keeps that until the copy is done),
+    so the call does not wait for the work queued before it as a copy from
+    pageable memory does; on another stream or device, or inside a capture,
+    each goes up synchronously."""
+    torch = _torch()
+    arrays = [None if v is None else np.atleast_1d(np.asarray(v, np.float32)) for v in values]
+    if stream is not None or device.index != torch._C._cuda_getDevice() or torch.cuda.is_current_stream_capturing():
+        return [None if a is None else torch.as_tensor(a, device=device) for a in arrays]
+    host = torch.empty(sum(a.size for a in arrays if a is not None), dtype=torch.float32, pin_memory=True)
+    flat, at, spans = host.numpy(), 0, []
+    for a in arrays:
+        size = 0 if a is None else a.size
+        flat[at:at + size] = 0 if a is None else a.ravel()
+        spans.append(None if a is None else (at, at + size))
+        at += size
+    dev = host.to(device, non_blocking=True)
+    return [None if sp is None else dev[sp[0]:sp[1]] for sp in spans]
+
+
 def quantize(x, scale, stream=None):
     """x [N,C,...] fp32 -> int8; scale: 1 or C values (per channel dim 1)."""
     torch = _torch()
     x = _dev(x, torch.float32)
     n, c = x.shape[0], x.shape[1]
     plane = x[0, 0].numel()
-    s = torch.as_tensor(np.atleast_1d(np.asarray(scale, np.float32)), device=x.device)
+    s, = _params(x.device, stream, scale)
     out = torch.empty(x.shape, dtype=torch.int8, device=x.device)
     check(load().nhip_quantize_f32_i8(_ptr(x), _ptr(out), n, c, plane, _ptr(s), s.numel(), _stream(stream)))
     return out
@@ -586,11 +612,8 @@ def requantize(x, in_scale, out_scale, bias=None, activation=ACT_NONE, stream=No
     x = _dev(x, torch.int32)
     n, c = x.shape[0], x.shape[1]
     plane = x[0, 0].numel()
-    dev = x.device
-    isc = torch.as_tensor(np.atleast_1d(np.asarray(in_scale, np.float32)), device=dev)
-    osc = torch.as_tensor(np.atleast_1d(np.asarray(out_scale, np.float32)), device=dev)
-    b = None if bias is None else torch.as_tensor(np.atleast_1d(np.asarray(bias, np.float32)), device=dev)
-    out = torch.empty(x.shape, dtype=torch.int8, device=dev)
+    isc, osc, b = _params(x.device, stream, in_scale, out_scale, bias)
+    out = torch.empty(x.shape, dtype=torch.int8, device=x.device)
     check(load().nhip_requantize_i32_i8(_ptr(x), _ptr(out), n, c, plane, _ptr(isc), isc.numel(), _ptr(osc),
                                         osc.numel(), _ptr(b), 0 if b is None else b.numel(), activation,
                                         _stream(stream)))
@@ -602,10 +625,8 @@ def dequantize(x, scale, bias=None, stream=None):
     x = _dev(x, torch.int32)
     n, c = x.shape[0], x.shape[1]
     plane = x[0, 0].numel()
-    dev = x.device
-    s = torch.as_tensor(np.atleast_1d(np.asarray(scale, np.float32)), device=dev)
-    b = None if bias is None else torch.as_tensor(np.atleast_1d(np.asarray(bias, np.float32)), device=dev)
-    out = torch.empty(x.shape, dtype=torch.float32, device=dev)
+    s, b = _params(x.device, stream, scale, bias)
+    out = torch.empty(x.shape, dtype=torch.float32, device=x.device)
     check(load().nhip_dequantize_i32_f32(_ptr(x), _ptr(out), n, c, plane, _ptr(s), s.numel(), _ptr(b),
                                          0 if b is None else b.numel(), _stream(stream)))
     return out
