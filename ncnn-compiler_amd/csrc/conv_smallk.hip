@@ -1,11 +1,12 @@
 // fp32 convolution with a short reduction and few output channels
-// (C*kh*kw <= 32, K <= 32): the stem of MobileNetV2-style networks, 3 -> 32
+// (C*kh*kw <= 32, K <= 64): the stem of MobileNetV2-style networks, 3 -> 32
 // channels, 3x3, stride 2 (ncnn Convolution, lowered by the reference
 // through tosa.conv2d: NCNNToTosa.cpp:1316-1529).
 //
 // Such a layer moves far more bytes than it computes (the 224x224 stem at
 // batch 32 writes 51 MB for 0.7 GFLOP), and its GEMM is one MFMA block high:
-// M = 32 output channels, K = the whole reduction.  A wave takes 32 output
+// M = 32 output channels (grid y: the second 32, gathering again), K = the
+// whole reduction.  A wave takes 32 output
 // pixels at a time as one v_mfma_f32_32x32x2_f32 block: A = the weights (the
 // lane's 8 or 16 values, loaded once), B = the input taps gathered straight
 // from memory (lane (n, h) loads tap 2s + h of pixel n for step s; padding
@@ -52,6 +53,7 @@ __global__ __launch_bounds__(kThreads) void conv_smallk_kernel(SmallkArgs a) {
   const int gw = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * kThreads + threadIdx.x) >> 6));  // global wave
   const int nw = (int)(gridDim.x * (kThreads / 64));
   if (gw >= a.nblk) return;  // uniform over the wave; no barrier below
+  const int m0 = 32 * blockIdx.y;  // first output channel
 
   // A operand of step s: W[k = l%32][2s + l/32]; the lane's tap 2s + l/32
   // as an element offset from the window's corner (c*H + dy)*W + dx and its
@@ -64,7 +66,7 @@ __global__ __launch_bounds__(kThreads) void conv_smallk_kernel(SmallkArgs a) {
   int toff[STEPS], tdy[STEPS], tdx[STEPS];
 #pragma unroll
   for (int s = 0; s < STEPS; ++s) {
-    wa[s] = a.w[li * a.ldw + 2 * s + lh];
+    wa[s] = a.w[(m0 + li) * a.ldw + 2 * s + lh];
     const int t = a.ktab[2 * s + lh];
     const int c = t >> 16, dy = (t >> 8) & 255, dx = t & 255;
     const bool live = c < a.C;
@@ -76,10 +78,10 @@ __global__ __launch_bounds__(kThreads) void conv_smallk_kernel(SmallkArgs a) {
     asm volatile("" : "+v"(toff[s]), "+v"(tdy[s]), "+v"(tdx[s]));
   }
 #pragma unroll
-  for (int r = 0; r < 16; ++r) bias[r] = a.bias[8 * (r >> 2) + 4 * lh + (r & 3)];
+  for (int r = 0; r < 16; ++r) bias[r] = a.bias[m0 + 8 * (r >> 2) + 4 * lh + (r & 3)];
   const uint32_t plane_bytes = (uint32_t)a.OHW * 4u;
-  const uint32_t lane_off = (uint32_t)(4 * lh) * plane_bytes;  // channel 4(l/32)
-  const int k_left = a.K - 4 * lh;                             // channels m < K: 8(r/4) + r%4 < k_left
+  const uint32_t lane_off = (uint32_t)(m0 + 4 * lh) * plane_bytes;  // channel m0 + 4(l/32)
+  const int k_left = a.K - m0 - 4 * lh;                             // channels m < K: 8(r/4) + r%4 < k_left
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, a.x_bytes);
   const __amdgpu_buffer_rsrc_t orr = make_rsrc(a.out, a.out_bytes);
   const __amdgpu_buffer_rsrc_t rr = make_rsrc(a.residual, RES ? a.out_bytes : 0u);
@@ -131,7 +133,7 @@ __global__ __launch_bounds__(kThreads) void conv_smallk_kernel(SmallkArgs a) {
     // of the channel bound are per lane, the register's part a multiple of
     // the plane size
     const uint32_t base = (uint32_t)((px.img * a.K) * a.OHW + px.q) * 4u + lane_off;
-    if (a.K == 32 && (blk + 1) * 32 <= a.npix) {
+    if (a.K - m0 >= 32 && (blk + 1) * 32 <= a.npix) {
       // every channel and pixel present: the register's part of the offset
       // goes in the instructions' scalar offset
       float res[16];
@@ -205,7 +207,7 @@ void launch_steps(const SmallkArgs& a, int act, dim3 grid, hipStream_t s) {
 }  // namespace
 
 // Shapes taken: a plain (groups 1) fp32 convolution on the implicit-GEMM
-// plan whose reduction is at most 32 long with at most 32 output channels,
+// plan whose reduction is at most 32 long with at most 64 output channels,
 // except 1x1 stride-1 unpadded ones (the pointwise kernels' shapes), and
 // 32-bit buffer offsets; by default only from four 32-pixel blocks per CU
 // (measured on the 224x224 stem: 26.4 against 35.7 us at batch 32, 11.1
@@ -218,7 +220,7 @@ bool smallk_supported(const nhip_conv_plan* p, int n, int h, int w, int oh, int 
   if (p->kind != PlanKind::ConvF32 || p->algorithm != NHIP_CONV_ALGO_IMPLICIT_GEMM) return false;
   const int mode = setting_int("NHIP_CONV_SMALLK", 1);
   if (mode == 0) return false;
-  if (p->kred > 32 || p->kred_pad > 32 || g.k > 32) return false;
+  if (p->kred > 32 || p->kred_pad > 32 || g.k > 64) return false;
   if (g.kh == 1 && g.kw == 1 && g.sh == 1 && g.sw == 1 && !g.pt && !g.pb && !g.pl && !g.pr) return false;
   const int64_t xb = (int64_t)n * g.c * h * w * 4, ob = (int64_t)n * g.k * oh * ow * 4;
   if (!(xb < (int64_t(1) << 31) && ob < (int64_t(1) << 31) && oh > 0 && ow > 0)) return false;
@@ -264,9 +266,11 @@ int launch_conv_smallk(const nhip_conv_plan* p, const float* in, const float* re
   // half of the SIMDs) 26.0 us, 768 29.7 us.  Two-block-deep and
   // three-block-deep gather rings were 1.2 and 2.3 us slower than the
   // one-block-ahead pair of buffers kept here.
-  const int per_cu = a.nblk >= 16LL * cu_count() ? 8 : 4;
-  const int64_t waves = std::min<int64_t>(a.nblk, (int64_t)per_cu * cu_count());
-  const dim3 grid((unsigned)ceil_div(waves, kThreads / 64));
+  // (The two halves of 33 to 64 channels share those waves.)
+  const int ny = (int)ceil_div(a.K, 32);
+  const int per_cu = ny * (int64_t)a.nblk >= 16LL * cu_count() ? 8 : 4;
+  const int64_t waves = std::min<int64_t>(a.nblk, (int64_t)per_cu / ny * cu_count());
+  const dim3 grid((unsigned)ceil_div(waves, kThreads / 64), (unsigned)ny);
   if (p->kred_pad <= 16) launch_steps<8>(a, p->g.act, grid, s);
   else launch_steps<16>(a, p->g.act, grid, s);
   return check_launch("conv_smallk_f32");

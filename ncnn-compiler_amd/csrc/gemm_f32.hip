@@ -1,23 +1,17 @@
-// fp32 MFMA GEMM core (v_mfma_f32_32x32x2_f32, wave64) and the two
-// contractions that use it (the Winograd batched GEMM has its own kernel in
-// wino_gemm.hip):
-//   - implicit-GEMM Convolution over NCHW blobs (reference ConvertConvolution
-//     fp32 path, NCNNToTosa.cpp:1316-1529, lowered upstream to
-//     linalg.conv_2d_nhwc_hwcf: out = bias + sum_{kh,kw,c} x*w);
-//   - InnerProduct (NCNNToTosa.cpp:5254-5392: zero-init matmul, then bias).
+// fp32 InnerProduct (NCNNToTosa.cpp:5254-5392: zero-init matmul, then bias) on
+// v_mfma_f32_32x32x2_f32, for inputs that the other InnerProduct kernels do not
+// take (not 16-byte aligned); the global-average-pooling + InnerProduct pair;
+// and the choice among the fp32 convolution kernels.
 //
-// GEMM view: D[i][j] = sum_k A[i][k] * B[k][j].  A rows i are output channels
-// (conv) or input rows m (InnerProduct); B columns j are output pixels or
-// InnerProduct outputs.  One workgroup = 4 waves
-// (2x2) computes a BM x BN tile; each wave a (BM/2) x (BN/2) tile built from
-// 32x32 MFMA blocks.  K advances in chunks of 16 through double-buffered LDS.
+// GEMM view: D[i][j] = sum_k A[i][k] * B[k][j], i an input row, j an output.
+// One workgroup = 4 waves (2x2) computes a 64 x 64 tile; each wave one 32x32
+// MFMA block.  K advances in chunks of 16 through double-buffered LDS.
 //
 // MFMA k mapping: in chunk-local step s (0..7) lane l supplies k = 8*(l/32)+s
 // for both operands, so each lane reads 8 consecutive k of its A row (two
 // ds_read_b128) instead of 16 scattered words.  Any permutation of k is valid
 // for a dot product as long as A and B use the same one.
-#include <cstdio>
-#include <cstdlib>
+#include <algorithm>
 
 #include "nhip_internal.h"
 
@@ -25,36 +19,25 @@ namespace nhip {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kBK = 16;      // K chunk of the MFMA k mapping; tiles use BK = 16 or 32
+constexpr int kBK = 16;     // K chunk of the MFMA k mapping
 constexpr int kRowPad = 4;  // LDS row padding (floats): conflict-free b128 reads
 constexpr int kXcds = 8;    // accelerator complex dies on MI355X
 
-enum class Mode { Conv, IP };
-
 struct GemmArgs {
-  // A operand
-  const float* a;        // conv: weights [m_pad][lda]; IP: input [M][lda]
+  const float* a;        // input [M][lda]
   int lda;
-  int m;                 // valid rows of the problem (out channels / IP rows)
-  // B operand
-  const float* b;        // conv: input NCHW; IP: W [n_pad][ldb]
+  int m;                 // input rows
+  const float* b;        // W [n_pad][ldb]
   int ldb;
-  int n;                 // valid columns (pixels / IP outputs)
-  int kdim;              // reduction length (multiple of BK after padding)
-  int k_valid;           // IP: valid input length (loads past it read 0)
-  uint32_t b_bytes;      // conv: size of the input tensor (< 2^31)
-  // conv geometry
-  const int* ktab;
-  int C, H, W, OW, OHW, sh, sw, pt, pl;
-  int pointwise;         // 1x1, stride 1, no padding: reduction index k is channel k (no ktab lookup)
-  // epilogue
-  float* d;              // conv: out NCHW; IP: out [M][ldd]
+  int n;                 // outputs
+  int kdim;              // reduction length (multiple of 16 after padding)
+  int k_valid;           // valid input length (loads past it read 0)
+  float* d;              // out [M][ldd], or raw partials [split][M][ldd]
   int ldd;
   const float* bias;
-  const float* residual;
   int act;
-  int splits;            // split-K factor (IP): >1 writes raw partials to d
-  int a_vec4;            // IP: lda % 4 == 0 (float4 A loads allowed)
+  int splits;            // split-K factor
+  int a_vec4;            // lda % 4 == 0 (float4 A loads allowed)
 };
 
 __device__ __forceinline__ float apply_act(float v, int act) {
@@ -63,26 +46,13 @@ __device__ __forceinline__ float apply_act(float v, int act) {
   return v;
 }
 
-template <int BM, int BN, int BK, Mode MODE>
-__global__ __launch_bounds__(kThreads) void gemm_f32_kernel(GemmArgs g) {
-  static_assert(BK % kBK == 0, "BK is a multiple of the 16-wide MFMA k chunk");
-  constexpr int TM = BM / 64;  // 32x32 blocks per wave along i
-  constexpr int TN = BN / 64;  // along j
-  constexpr int AS = BK + kRowPad;                  // As[BM][AS], Bs[BN][AS]
-  constexpr int B_ELEMS = BN * AS;
-  // One LDS array: two A and two B operand buffers, reused by the conv
-  // epilogue for a 64 x (BN+4) staging slab.
-  constexpr int OPER = 2 * (BM * AS + B_ELEMS);
-  constexpr int SLAB = (MODE == Mode::Conv) ? 64 * (BN + 4) : 0;
-  __shared__ __attribute__((aligned(16))) float smem[OPER > SLAB ? OPER : SLAB];
+__global__ __launch_bounds__(kThreads) void gemm_ip_kernel(GemmArgs g) {
+  constexpr int BM = 64, BN = 64, AS = kBK + kRowPad;  // As[BM][AS], Bs[BN][AS]
+  __shared__ __attribute__((aligned(16))) float smem[2 * (BM + BN) * AS];
   auto As = [&](int buf) { return smem + buf * BM * AS; };
-  auto Bs = [&](int buf) { return smem + 2 * BM * AS + buf * B_ELEMS; };
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int li = lane & 31, lh = lane >> 5;
+  auto Bs = [&](int buf) { return smem + 2 * BM * AS + buf * BN * AS; };
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1, li = lane & 31, lh = lane >> 5;
 
   // Workgroups are dispatched round-robin over the XCDs (8 on MI355X, each
   // with its own L2): hardware id L runs on XCD L % 8.  Renumber so that each
@@ -99,162 +69,54 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_kernel(GemmArgs g) {
     by = (logical / nbx) % nby;
     bz = logical / (nbx * nby);
   }
-  const int j0 = bx * BN;
-  const int i0 = by * BM;
-  const int split = bz;  // K split (grid z)
-
-  const float* A = g.a;
-  const float* B = g.b;
-
-  const int nk_total = g.kdim / BK;
+  const int j0 = bx * BN, i0 = by * BM;
+  const int nk_total = g.kdim / kBK;
   const int per = (nk_total + g.splits - 1) / g.splits;
-  const int kt_begin = min(nk_total, split * per);
-  const int kt_end = min(nk_total, kt_begin + per);
+  const int kt_begin = min(nk_total, bz * per), kt_end = min(nk_total, kt_begin + per);
 
-  // ---- operand stages.  A: BM x BK floats as float4 rows.  B (Conv): im2col
-  // gather, thread owns pixel column jj = tid % BN and KPT consecutive k
-  // (KPT = BK*BN/256).  B (IP): W [j][k] rows, like A.
-  constexpr int A_Q = BK / 4;  // float4 per A row chunk
-  constexpr int A_LD = BM * A_Q / kThreads;
-  constexpr int KPT = BK * BN / kThreads;
-  constexpr int B_LD4 = BN * A_Q / kThreads;
-  // Native vectors: HIP's float4 struct copies would keep a stage in scratch.
+  // a thread's operand of a stage: 4 consecutive k of one row of each
   struct Stage {
-    v4f a[A_LD];
-    float b[(MODE == Mode::Conv) ? KPT : 1];
-    v4f b4[(MODE == Mode::Conv) ? 1 : B_LD4];
+    v4f a, b;
   };
-
-  // Conv per-thread pixel state (fixed for the whole block).
-  const int jj = tid % BN;
-  const int kg = __builtin_amdgcn_readfirstlane(tid / BN);
-  // Conv: the whole input is one wave-uniform buffer resource (< 2^31 bytes);
-  // zero padding reads through kBufOOB offsets.
-  const __amdgpu_buffer_rsrc_t img_rs = make_rsrc(B, g.b_bytes);
-  int iy0 = 0, ix0 = 0, img_plane0 = 0;
-  bool pix_ok = false;
-  if constexpr (MODE == Mode::Conv) {
-    const int p = j0 + jj;
-    pix_ok = p < g.n;
-    const int pp = pix_ok ? p : 0;
-    const int img = pp / g.OHW;
-    const int rem = pp - img * g.OHW;
-    const int oh = rem / g.OW;
-    const int ow = rem - oh * g.OW;
-    iy0 = oh * g.sh - g.pt;
-    ix0 = ow * g.sw - g.pl;
-    img_plane0 = img * g.C;
-  }
-
+  const int row = tid / 4, kq = (tid % 4) * 4;
   auto gload = [&](Stage& st, int kt) {
-#pragma unroll
-    for (int u = 0; u < A_LD; ++u) {
-      const int q = tid + u * kThreads;
-      const int row = q / A_Q, kq = (q % A_Q) * 4;
-      const int k = kt * BK + kq;
-      if constexpr (MODE == Mode::IP) {
-        const int r = i0 + row;
-        v4f v = {0.f, 0.f, 0.f, 0.f};
-        if (r < g.m) {
-          const float* src = A + (int64_t)r * g.lda;
-          if (g.a_vec4) {
-            if (k < g.k_valid) v = *reinterpret_cast<const v4f*>(src + k);
-          } else {
-            v.x = (k + 0 < g.k_valid) ? src[k + 0] : 0.f;
-            v.y = (k + 1 < g.k_valid) ? src[k + 1] : 0.f;
-            v.z = (k + 2 < g.k_valid) ? src[k + 2] : 0.f;
-            v.w = (k + 3 < g.k_valid) ? src[k + 3] : 0.f;
-          }
-        }
-        st.a[u] = v;
+    const int k = kt * kBK + kq, r = i0 + row;
+    v4f v = {0.f, 0.f, 0.f, 0.f};
+    if (r < g.m) {
+      const float* src = g.a + (int64_t)r * g.lda;
+      if (g.a_vec4) {
+        if (k < g.k_valid) v = *reinterpret_cast<const v4f*>(src + k);
       } else {
-        st.a[u] = *reinterpret_cast<const v4f*>(A + (int64_t)(i0 + row) * g.lda + k);
+        v.x = (k + 0 < g.k_valid) ? src[k + 0] : 0.f;
+        v.y = (k + 1 < g.k_valid) ? src[k + 1] : 0.f;
+        v.z = (k + 2 < g.k_valid) ? src[k + 2] : 0.f;
+        v.w = (k + 3 < g.k_valid) ? src[k + 3] : 0.f;
       }
     }
-    if constexpr (MODE == Mode::Conv) {
-      const int kbase = kt * BK + kg * KPT;
-#pragma unroll
-      for (int u = 0; u < KPT; ++u) {
-        int c = kbase + u, dy = 0, dx = 0;
-        if (!g.pointwise) {  // wave-uniform table entry
-          const int t = g.ktab[kbase + u];
-          c = t >> 16;
-          dy = (t >> 8) & 255;
-          dx = t & 255;
-        }
-        const int y = iy0 + dy, x = ix0 + dx;
-        const bool in = pix_ok && c < g.C && (unsigned)y < (unsigned)g.H && (unsigned)x < (unsigned)g.W;
-        st.b[u] = buf_load_f32(img_rs, in ? (uint32_t)((((img_plane0 + c) * g.H + y) * g.W + x) * (int)sizeof(float))
-                                          : kBufOOB);
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < B_LD4; ++u) {
-        const int q = tid + u * kThreads;
-        const int row = q / A_Q, kq = (q % A_Q) * 4;
-        st.b4[u] = *reinterpret_cast<const v4f*>(B + (int64_t)(j0 + row) * g.ldb + kt * BK + kq);
-      }
-    }
+    st.a = v;
+    st.b = *reinterpret_cast<const v4f*>(g.b + (int64_t)(j0 + row) * g.ldb + k);
   };
   auto lstore = [&](const Stage& st, int buf) {
-#pragma unroll
-    for (int u = 0; u < A_LD; ++u) {
-      const int q = tid + u * kThreads;
-      const int row = q / A_Q, kq = (q % A_Q) * 4;
-      *reinterpret_cast<v4f*>(&As(buf)[row * AS + kq]) = st.a[u];
-    }
-    if constexpr (MODE == Mode::Conv) {
-#pragma unroll
-      for (int u = 0; u < KPT; u += 4)
-        *reinterpret_cast<v4f*>(&Bs(buf)[jj * AS + kg * KPT + u]) = v4f{st.b[u], st.b[u + 1], st.b[u + 2], st.b[u + 3]};
-    } else {
-#pragma unroll
-      for (int u = 0; u < B_LD4; ++u) {
-        const int q = tid + u * kThreads;
-        const int row = q / A_Q, kq = (q % A_Q) * 4;
-        *reinterpret_cast<v4f*>(&Bs(buf)[row * AS + kq]) = st.b4[u];
-      }
-    }
+    *reinterpret_cast<v4f*>(&As(buf)[row * AS + kq]) = st.a;
+    *reinterpret_cast<v4f*>(&Bs(buf)[row * AS + kq]) = st.b;
   };
 
-  v16f acc[TM][TN];
+  v16f acc;
 #pragma unroll
-  for (int a = 0; a < TM; ++a)
-#pragma unroll
-    for (int b = 0; b < TN; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.f;
-
+  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   auto compute = [&](int buf) {
+    const float* pa = &As(buf)[(wm * 32 + li) * AS + lh * 8];
+    const float* pb = &Bs(buf)[(wn * 32 + li) * AS + lh * 8];
+    const v4f a0 = *reinterpret_cast<const v4f*>(pa), a1 = *reinterpret_cast<const v4f*>(pa + 4);
+    const v4f b0 = *reinterpret_cast<const v4f*>(pb), b1 = *reinterpret_cast<const v4f*>(pb + 4);
 #pragma unroll
-    for (int kc = 0; kc < BK; kc += kBK) {
-      v4f af[TM][2], bf[TN][2];
+    for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[s], b0[s], acc, 0, 0, 0);
 #pragma unroll
-      for (int a = 0; a < TM; ++a) {
-        const float* pa = &As(buf)[(wm * (BM / 2) + a * 32 + li) * AS + kc + lh * 8];
-        af[a][0] = *reinterpret_cast<const v4f*>(pa);
-        af[a][1] = *reinterpret_cast<const v4f*>(pa + 4);
-      }
-#pragma unroll
-      for (int b = 0; b < TN; ++b) {
-        const float* pb = &Bs(buf)[(wn * (BN / 2) + b * 32 + li) * AS + kc + lh * 8];
-        bf[b][0] = *reinterpret_cast<const v4f*>(pb);
-        bf[b][1] = *reinterpret_cast<const v4f*>(pb + 4);
-      }
-#pragma unroll
-      for (int s = 0; s < 8; ++s)
-#pragma unroll
-        for (int a = 0; a < TM; ++a)
-#pragma unroll
-          for (int b = 0; b < TN; ++b)
-            acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[a][s >> 2][s & 3], bf[b][s >> 2][s & 3], acc[a][b],
-                                                             0, 0, 0);
-    }
+    for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[s], b1[s], acc, 0, 0, 0);
   };
 
   // Two LDS buffers, global loads two stages ahead; the loop body is
-  // straight-line (two stages per trip, odd tail peeled) so the accumulators
-  // keep one register range.
+  // straight-line (two stages per trip, odd tail peeled).
   const int n = kt_end - kt_begin;
   if (n > 0) {
     Stage s0, s1;
@@ -276,125 +138,19 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_kernel(GemmArgs g) {
     if (i < n) compute(0);
   }
 
-  // ---- epilogue.  32x32 accumulator layout: register r of lane l holds
-  // row (r%4) + 8*(r/4) + 4*(l/32), column l%32.
-  if constexpr (MODE == Mode::Conv) {
-    if (g.splits == 1) {
-      // Staged through LDS one 64-row slab (a) at a time: each thread then
-      // writes runs of 4 pixels of one output channel with 16-byte accesses
-      // (bias once per run, residual read as a vector), 32-bit offsets (a
-      // launch's tensors stay below 2^31 bytes).  Same order as the direct
-      // epilogue: acc + bias, + residual, then the activation.
-      constexpr int TS = BN + 4;  // staged row stride (floats)
-      float* tile = smem;
-      const int ohw = g.OHW;
-      const bool vec = (ohw & 3) == 0;
+  // 32x32 accumulator layout: register r of lane l holds row (r%4) + 8*(r/4) +
+  // 4*(l/32), column l%32.
+  const int j = j0 + wn * 32 + li;
+  if (j >= g.n) return;
 #pragma unroll
-      for (int a = 0; a < TM; ++a) {
-        __syncthreads();
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            tile[(wm * 32 + (r & 3) + 8 * (r >> 2) + 4 * lh) * TS + wn * (BN / 2) + b * 32 + li] = acc[a][b][r];
-        __syncthreads();
-        for (int q = tid; q < 64 * (BN / 4); q += kThreads) {
-          const int lr = q / (BN / 4), lc = (q % (BN / 4)) * 4;
-          const int i = i0 + (lr >> 5) * (BM / 2) + a * 32 + (lr & 31);
-          const int j = j0 + lc;
-          if (i >= g.m || j >= g.n) continue;
-          const float bi = g.bias[i];
-          const int img = j / ohw, rem = j - img * ohw;
-          const int o = (img * g.m + i) * ohw + rem;
-          const v4f t = *reinterpret_cast<const v4f*>(&tile[lr * TS + lc]);
-          if (vec && j + 4 <= g.n) {  // a 4-run never crosses an image when ohw % 4 == 0
-            v4f v = t + bi;
-            if (g.residual) v += *reinterpret_cast<const v4f*>(g.residual + o);
-            v.x = apply_act(v.x, g.act);
-            v.y = apply_act(v.y, g.act);
-            v.z = apply_act(v.z, g.act);
-            v.w = apply_act(v.w, g.act);
-            *reinterpret_cast<v4f*>(g.d + o) = v;
-          } else {
-            for (int e = 0; e < 4 && j + e < g.n; ++e) {
-              const int je = j + e, ie = je / ohw;
-              const int oe = (ie * g.m + i) * ohw + (je - ie * ohw);
-              float v = t[e] + bi;
-              if (g.residual) v += g.residual[oe];
-              g.d[oe] = apply_act(v, g.act);
-            }
-          }
-        }
-      }
-      return;
-    }
+  for (int r = 0; r < 16; ++r) {
+    const int i = i0 + wm * 32 + (r & 3) + 8 * (r >> 2) + 4 * lh;
+    if (i >= g.m) continue;
+    if (g.splits > 1)
+      g.d[((int64_t)bz * g.m + i) * g.ldd + j] = acc[r];
+    else
+      g.d[(int64_t)i * g.ldd + j] = apply_act(acc[r] + g.bias[j], g.act);
   }
-#pragma unroll
-  for (int b = 0; b < TN; ++b) {
-    const int j = j0 + wn * (BN / 2) + b * 32 + li;
-    if constexpr (MODE == Mode::Conv) {
-      if (j >= g.n) continue;
-      if (g.splits > 1) {  // raw partial sums [split][m][n]; bias etc. in conv_splitk_reduce
-        float* P = g.d + (int64_t)split * g.m * g.n;
-#pragma unroll
-        for (int a = 0; a < TM; ++a)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int i = i0 + wm * (BM / 2) + a * 32 + (r & 3) + 8 * (r >> 2) + 4 * lh;
-            if (i < g.m) P[(int64_t)i * g.n + j] = acc[a][b][r];
-          }
-        continue;
-      }
-      const int img = j / g.OHW;
-      const int rem = j - img * g.OHW;
-      const int64_t obase = (int64_t)img * g.m * g.OHW + rem;
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int i = i0 + wm * (BM / 2) + a * 32 + (r & 3) + 8 * (r >> 2) + 4 * lh;
-          if (i < g.m) {
-            const int64_t o = obase + (int64_t)i * g.OHW;
-            float v = acc[a][b][r] + g.bias[i];
-            if (g.residual) v += g.residual[o];
-            g.d[o] = apply_act(v, g.act);
-          }
-        }
-    } else {
-      if (j >= g.n) continue;
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int i = i0 + wm * (BM / 2) + a * 32 + (r & 3) + 8 * (r >> 2) + 4 * lh;
-          if (i < g.m) {
-            if (g.splits > 1) {
-              g.d[((int64_t)split * g.m + i) * g.ldd + j] = acc[a][b][r];
-            } else {
-              g.d[(int64_t)i * g.ldd + j] = apply_act(acc[a][b][r] + g.bias[j], g.act);
-            }
-          }
-        }
-    }
-  }
-}
-
-// Split-K reduction for the implicit-GEMM convolution: part [S][m][npix] ->
-// out NCHW = act(sum_s part + bias (+ residual)), the order of the unsplit
-// epilogue.
-__global__ void conv_splitk_reduce(const float* __restrict__ part, int splits, int m, int npix, int ohw,
-                                   const float* __restrict__ bias, const float* __restrict__ residual,
-                                   float* __restrict__ out, int act) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)m * npix) return;
-  const int i = (int)(idx / npix), j = (int)(idx - (int64_t)i * npix);
-  float acc = part[idx];
-  for (int s = 1; s < splits; ++s) acc += part[(int64_t)s * m * npix + idx];
-  const int img = j / ohw, rem = j - img * ohw;
-  const int64_t o = ((int64_t)img * m + i) * ohw + rem;
-  float v = acc + bias[i];
-  if (residual) v += residual[o];
-  out[o] = apply_act(v, act);
 }
 
 // Split-K reduction for InnerProduct: out = act((sum_s part[s]) + bias).
@@ -420,53 +176,32 @@ __global__ void ip_splitk_reduce(const float* part, const float* bias,
   out[idx] = apply_act(s + bias[j], act);
 }
 
-template <int BM, int BN, Mode MODE, int BK = kBK>
-int launch(const GemmArgs& g, dim3 grid, hipStream_t s, const char* name) {
-  NHIP_LAUNCH(name, (gemm_f32_kernel<BM, BN, BK, MODE>), grid, dim3(kThreads), 0, s, g);
-  return check_launch(name);
-}
-
 }  // namespace
 
 // ------------------------------- Convolution ------------------------------
-namespace {
-struct IgemmCfg {
-  int bm, bn, splits;
-};
-// Tile: the largest that still gives about two workgroups per CU (64x64
-// otherwise).  K split: when even that leaves the CUs short of work and K is
-// long, split K so that each workgroup keeps at least 4 chunks.
-IgemmCfg igemm_config(const nhip_conv_plan* p, int64_t npix) {
-  const int64_t target = 2LL * cu_count();
-  const int64_t mt128 = ceil_div(p->g.k, 128), mt64 = ceil_div(p->g.k, 64);
-  const int64_t nt128 = ceil_div(npix, 128);
-  IgemmCfg c{64, 64, 1};
-  // Short reductions (1x1 and stem convolutions, K <= 256) are bandwidth-bound:
-  // the 64x64 tile gives the most workgroups and measures fastest there.
-  if (p->kred_pad > 256) {
-    if (p->m_pad % 128 == 0 && mt128 * nt128 >= target) c = {128, 128, 1};
-    else if (mt64 * nt128 >= target) c = {64, 128, 1};
-  }
-  // Tuning override NHIP_IGEMM_TILE="bm,bn" (64x64, 64x128, 128x128).
-  if (const char* env = setting("NHIP_IGEMM_TILE")) {
-    int bm = 0, bn = 0;
-    if (std::sscanf(env, "%d,%d", &bm, &bn) == 2 && (bm == 64 || (bm == 128 && p->m_pad % 128 == 0)) &&
-        (bn == 64 || bn == 128) && !(bm == 128 && bn == 64))
-      c = {bm, bn, 1};
-  }
-  const int64_t tiles = ceil_div(p->g.k, c.bm) * ceil_div(npix, c.bn);
-  const int nk = p->kred_pad / kBK;
-  while (c.splits < 16 && tiles * c.splits < cu_count() && nk / (c.splits * 2) >= 4) c.splits *= 2;
-  return c;
+// A 1x1 stride-1 layer that runs faster on the split kernel than on the
+// streaming 1x1 kernel, both measured: from 176 input channels on (288 -> 80,
+// 15488 pixels: 17.9 -> 15.8 us; 448 -> 368, 6498: 37.3 -> 26.9; 168 -> 48,
+// 4356: 6.0 against 6.6), and from 48 where the planes are no multiple of four
+// pixels, which the streaming kernel reads one element at a time (80 -> 240,
+// 57x57 x 2: 15.1 -> 11.0; 24 -> 264, 22x22: no difference).  Up to 32768 pixels:
+// launches beyond stream more than the caches hold, and there the streaming
+// kernel's 16-byte loads win (192 -> 96, 50176 pixels: 25.3 against 29.6; 200
+// -> 40, 100352: 28.0 against 33.9; 256 -> 128, 25088: 25.4 -> 22.0).  A forced
+// 1x1 kernel (any NHIP_* switch of those kernels) is left alone.
+static bool split_1x1_preferred(const nhip_conv_plan* p, int n, int oh, int ow) {
+  for (const char* name : {"NHIP_POINTWISE", "NHIP_PW_CFG", "NHIP_PW_WGS", "NHIP_GEMM_DMA", "NHIP_CONV_KQ"})
+    if (setting(name)) return false;
+  const int64_t plane = (int64_t)oh * ow;
+  return n * plane < 32768 && (p->g.c >= 176 || (p->g.c >= 48 && plane % 4 != 0));
 }
-}  // namespace
 
 uint64_t conv_igemm_f32_workspace(const nhip_conv_plan* p, int n, int oh, int ow) {
-  if (pointwise_selected(p, n, oh, ow)) return 0;
-  if (pw_dma_supported(p, n, oh, ow)) return conv_pw_dma_workspace(p, n, oh, ow);
-  const int64_t npix = (int64_t)n * oh * ow;
-  const IgemmCfg c = igemm_config(p, npix);
-  return c.splits > 1 ? (uint64_t)c.splits * p->g.k * npix * sizeof(float) : 0;
+  if (!split_1x1_preferred(p, n, oh, ow)) {
+    if (pointwise_selected(p, n, oh, ow)) return 0;
+    if (pw_dma_supported(p, n, oh, ow)) return conv_pw_dma_workspace(p, n, oh, ow);
+  }
+  return conv_split_workspace(p, n, oh, ow);
 }
 
 int launch_conv_igemm_f32(const nhip_conv_plan* p, const float* in,
@@ -474,58 +209,14 @@ int launch_conv_igemm_f32(const nhip_conv_plan* p, const float* in,
                           int w, int oh, int ow, void* ws, uint64_t ws_bytes,
                           hipStream_t s) {
   // (the short-reduction kernel needs no workspace; the size query above
-  // keeps the implicit GEMM's, which is then unused)
+  // keeps the split kernel's, which is then unused)
   if (smallk_supported(p, n, h, w, oh, ow)) return launch_conv_smallk(p, in, residual, out, n, h, w, oh, ow, s);
   if (kq_supported(p, n, h, w, oh, ow)) return launch_conv_kq(p, in, residual, out, n, h, w, oh, ow, s);
-  if (pointwise_selected(p, n, h, w)) return launch_conv_pointwise_f32(p, in, residual, out, n, h, w, s);
-  if (pw_dma_supported(p, n, h, w)) return launch_conv_pw_dma(p, in, residual, out, n, h, w, ws, ws_bytes, s);
-  GemmArgs g{};
-  g.a = p->weight;
-  g.lda = p->kred_pad;
-  g.m = p->g.k;
-  g.b = in;
-  g.b_bytes = (uint32_t)((size_t)n * p->g.c * h * w * sizeof(float));
-  g.n = n * oh * ow;
-  g.kdim = p->kred_pad;
-  g.ktab = p->ktab;
-  g.C = p->g.c;
-  g.H = h;
-  g.W = w;
-  g.OW = ow;
-  g.OHW = oh * ow;
-  g.sh = p->g.sh;
-  g.sw = p->g.sw;
-  g.pt = p->g.pt;
-  g.pl = p->g.pl;
-  g.pointwise = p->g.kh == 1 && p->g.kw == 1 && p->g.sh == 1 && p->g.sw == 1 && p->g.pt == 0 && p->g.pl == 0 &&
-                p->g.pb == 0 && p->g.pr == 0;
-  g.d = out;
-  g.bias = p->bias;
-  g.residual = residual;
-  g.act = p->g.act;
-  const IgemmCfg c = igemm_config(p, g.n);
-  g.splits = c.splits;
-  if (c.splits > 1) {
-    const uint64_t need = conv_igemm_f32_workspace(p, n, oh, ow);
-    if (ws == nullptr || ws_bytes < need)
-      return fail(NHIP_STATUS_OUTPUT_CAPACITY_INSUFFICIENT,
-                  "implicit-GEMM conv: workspace of " + std::to_string(need) + " bytes required");
-    g.d = static_cast<float*>(ws);
+  if (!split_1x1_preferred(p, n, oh, ow)) {
+    if (pointwise_selected(p, n, h, w)) return launch_conv_pointwise_f32(p, in, residual, out, n, h, w, s);
+    if (pw_dma_supported(p, n, h, w)) return launch_conv_pw_dma(p, in, residual, out, n, h, w, ws, ws_bytes, s);
   }
-  const dim3 grid((unsigned)ceil_div(g.n, c.bn), (unsigned)ceil_div(p->g.k, c.bm), (unsigned)c.splits);
-  if (c.bm == 128)
-    NHIP_TRY((launch<128, 128, Mode::Conv>(g, grid, s, "conv_igemm_f32<128,128>")));
-  else if (c.bn == 128)
-    NHIP_TRY((launch<64, 128, Mode::Conv>(g, grid, s, "conv_igemm_f32<64,128>")));
-  else
-    NHIP_TRY((launch<64, 64, Mode::Conv>(g, grid, s, "conv_igemm_f32<64,64>")));
-  if (c.splits > 1) {
-    const int64_t total = (int64_t)p->g.k * g.n;
-    NHIP_LAUNCH("conv_splitk_reduce", conv_splitk_reduce, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, s,
-                static_cast<const float*>(ws), c.splits, p->g.k, g.n, g.OHW, p->bias, residual, out, p->g.act);
-    return check_launch("conv_splitk_reduce");
-  }
-  return ok();
+  return launch_conv_split(p, in, residual, out, n, h, w, oh, ow, ws, ws_bytes, s);
 }
 
 // ------------------------------- InnerProduct -----------------------------
@@ -726,8 +417,9 @@ int launch_innerproduct_f32(const nhip_ip_plan* p, const float* in,
   }
   // B rows (weights) are padded to n_pad (multiple of 64); j bounds are
   // checked in the epilogue only.
-  NHIP_TRY((launch<64, 64, Mode::IP>(g, dim3(p->n_pad / 64, (int)ceil_div(m, 64), splits), s,
-                                     "innerproduct_f32<64,64>")));
+  NHIP_LAUNCH("innerproduct_f32<64,64>", gemm_ip_kernel, dim3(p->n_pad / 64, (int)ceil_div(m, 64), splits),
+              dim3(kThreads), 0, s, g);
+  NHIP_TRY(check_launch("innerproduct_f32<64,64>"));
   if (splits > 1) {
     const int64_t total = (int64_t)m * p->n_out;
     NHIP_LAUNCH("ip_splitk_reduce", ip_splitk_reduce, dim3((unsigned)ceil_div(total, 256)), dim3(256), 0, s,

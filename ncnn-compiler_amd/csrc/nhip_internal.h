@@ -176,15 +176,20 @@ struct nhip_conv_plan {
   // the 32 output channels of one group are contiguous.
   float* weight_kq = nullptr;
   int32_t kq_vw = 0;
-  // Winograd plans of 256+ input channels: an implicit-GEMM plan of the same
-  // layer, for launches of so few tiles that the Winograd GEMM's 128-tile
-  // padding dominates (a single 7x7 or 14x14 image).
-  nhip_conv_plan* igemm_twin = nullptr;
   // 1x1 plans with at most 32 output channels: the weights channel-major,
   // [C][32] (zero past K), the LDS layout of the depthwise -> 1x1 kernel.
   float* weight_ck = nullptr;
   // 3x3 depthwise plans: [C][12], the nine taps, the bias, two zeros.
   float* weight_dw12 = nullptr;
+  // The weights split into three bf16 pieces in MFMA fragment order
+  // (conv_split.hip), [m_pad/32][split_nk][3][64 lanes][8], and where the fp32
+  // weights [K][split_ldw] in (c, kh, kw) order are (in the same buffer, or
+  // `weight`): implicit-GEMM plans, and Winograd plans for the launches that
+  // leave the Winograd kernels.
+  uint16_t* weight_split = nullptr;
+  const float* split_f32 = nullptr;
+  int32_t split_nk = 0, split_c_pad = 0, split_taps = 0, split_ldw = 0;
+  int32_t wino_auto = 0;      // Winograd chosen by the library, not by the caller
   float* bias = nullptr;      // [m_pad] zero-filled past k (always present)
   int32_t m_pad = 0, kred = 0, kred_pad = 0, c_pad = 0;
   // im2col gather table: one packed int per reduction index
@@ -224,7 +229,8 @@ namespace nhip {
 // Reduction length (bytes) of the int8 register-weight kernel: 36 k steps of
 // 32 bytes (128 channels at 3x3).
 constexpr int kRwKred = 36 * 32;
-// Input channels from which a Winograd plan also holds an implicit-GEMM twin.
+// Input channels from which a Winograd plan that the caller asked for still
+// leaves the Winograd kernels for launches of a few tiles.
 constexpr int kWinoTwinMinC = 256;
 // Kernel launchers (defined in the .hip files).
 int launch_conv_igemm_f32(const nhip_conv_plan* p, const float* in,
@@ -255,6 +261,12 @@ int launch_dwpw_f32(const nhip_conv_plan* dw, const nhip_conv_plan* pw, const fl
 bool dwpw_lds_supported(const nhip_conv_plan* dw, const nhip_conv_plan* pw, int n, int h, int w, int oh, int ow);
 int launch_dwpw_lds_f32(const nhip_conv_plan* dw, const nhip_conv_plan* pw, const float* in,
                         const float* residual, float* out, int n, int h, int w, int oh, int ow, hipStream_t s);
+// conv_split.hip: implicit GEMM on the bf16 matrix instructions, the fp32
+// operands split exactly into three bf16 pieces (any fp32 convolution).
+int conv_split_prepack(nhip_conv_plan* p, const float* weight, bool keep_f32);
+uint64_t conv_split_workspace(const nhip_conv_plan* p, int n, int oh, int ow);
+int launch_conv_split(const nhip_conv_plan* p, const float* in, const float* residual, float* out, int n, int h,
+                      int w, int oh, int ow, void* ws, uint64_t ws_bytes, hipStream_t s);
 int launch_conv_winograd_f32(const nhip_conv_plan* p, const float* in,
                              const float* residual, float* out, int n, int h,
                              int w, int oh, int ow, void* ws,

@@ -345,10 +345,10 @@ int upload_bias(nhip_conv_plan* p, const float* bias, int count, int padded) {
 
 void free_plan(nhip_conv_plan* p) {
   if (!p) return;
-  free_plan(p->igemm_twin);
   (void)hipFree(p->weight);
   (void)hipFree(p->weight_fused);
   (void)hipFree(p->weight_kq);
+  (void)hipFree(p->weight_split);
   (void)hipFree(p->weight_ck);
   (void)hipFree(p->weight_dw12);
   (void)hipFree(p->bias);
@@ -558,26 +558,31 @@ int nhip_conv2d_f32_create(const nhip_conv_desc* d, const float* weight, const f
     p->c_pad = (int)round_up(C, 16);
     st = winograd_prepack_weights(p, weight);
     if (st == NHIP_STATUS_SUCCESS) st = conv_kq_prepack(p, weight, C, K, 3, 3);
-    if (st == NHIP_STATUS_SUCCESS && C >= kWinoTwinMinC) {
-      nhip_conv_desc d2 = *d;
-      d2.algorithm = NHIP_CONV_ALGO_IMPLICIT_GEMM;
-      st = nhip_conv2d_f32_create(&d2, weight, bias, &p->igemm_twin);
-    }
+    p->wino_auto = d->algorithm == NHIP_CONV_ALGO_AUTO;
+    if (st == NHIP_STATUS_SUCCESS && (p->wino_auto || C >= kWinoTwinMinC)) st = conv_split_prepack(p, weight, true);
   } else {
     const int khw = d->kernel_h * d->kernel_w;
     p->kred = C * khw;
     p->kred_pad = (int)round_up(p->kred, 16);
-    std::vector<float> wp((size_t)p->m_pad * p->kred_pad, 0.f);
-    for (int k = 0; k < K; ++k)
-      std::copy(weight + (size_t)k * p->kred, weight + (size_t)(k + 1) * p->kred, wp.begin() + (size_t)k * p->kred_pad);
-    std::vector<int32_t> kt((size_t)p->kred_pad, 0x7fff << 16);
-    for (int k = 0; k < p->kred; ++k) {
-      const int c = k / khw, r = k % khw, kh = r / d->kernel_w, kw = r % d->kernel_w;
-      kt[k] = (c << 16) | ((kh * d->dilation_h) << 8) | (kw * d->dilation_w);
+    // row-major weights: the 1x1 kernels and the short-reduction one; the
+    // others hold them with the split ones
+    const bool rows = khw == 1 || (p->kred <= 32 && K <= 64);
+    if (rows) {
+      std::vector<float> wp((size_t)p->m_pad * p->kred_pad, 0.f);
+      for (int k = 0; k < K; ++k)
+        std::copy(weight + (size_t)k * p->kred, weight + (size_t)(k + 1) * p->kred, wp.begin() + (size_t)k * p->kred_pad);
+      st = upload(&p->weight, wp, "hipMalloc(conv weight)");
     }
-    st = upload(&p->weight, wp, "hipMalloc(conv weight)");
-    if (st == NHIP_STATUS_SUCCESS) st = upload(&p->ktab, kt, "hipMalloc(conv ktab)");
+    if (st == NHIP_STATUS_SUCCESS && (rows || 3 * round_up(C, 8) > 4 * C)) {  // read in (c, kh, kw) order
+      std::vector<int32_t> kt((size_t)p->kred_pad, 0x7fff << 16);
+      for (int k = 0; k < p->kred; ++k) {
+        const int c = k / khw, r = k % khw, kh = r / d->kernel_w, kw = r % d->kernel_w;
+        kt[k] = (c << 16) | ((kh * d->dilation_h) << 8) | (kw * d->dilation_w);
+      }
+      st = upload(&p->ktab, kt, "hipMalloc(conv ktab)");
+    }
     if (st == NHIP_STATUS_SUCCESS) st = conv_kq_prepack(p, weight, C, K, d->kernel_h, d->kernel_w);
+    if (st == NHIP_STATUS_SUCCESS) st = conv_split_prepack(p, weight, !rows);
     if (st == NHIP_STATUS_SUCCESS && khw == 1 && K <= 32) {
       std::vector<float> ck((size_t)C * 32, 0.f);
       for (int k = 0; k < K; ++k)

@@ -289,20 +289,25 @@ int winograd_prepack_weights(nhip_conv_plan* p, const float* weight) {
                    "hipMemcpy(winograd U)");
 }
 
-// Launches of at most 32 tiles on a plan with an implicit-GEMM twin take the
-// twin: the Winograd GEMM pads the tiles to 128, and a single image of
-// 512@7 (4 tiles) took 46.6 us on it against 23.3 us on the implicit GEMM,
-// 256@14 22.8 against 17.0 us at one image (16 tiles) and 23.3 against 21.8
-// at two (32 tiles), where from 64 tiles on Winograd wins (23.9 against
-// 29.4).  Not when a Winograd variant is forced (NHIP_WINOGRAD_VARIANT);
+// Launches that leave the Winograd kernels for the split implicit GEMM
+// (conv_split.hip).  The Winograd path costs 12 us (three launches) to 20 us
+// at the least, whatever its size, and its GEMM pads the tiles to 128; the
+// split kernel takes 6 us plus about 10 us per GFLOP of the direct
+// convolution.  Plans whose algorithm the library chose: up to 1.5 GFLOP
+// (9 x 40 -> 24 @ 21x21, 0.07 GFLOP: 19.8 -> 6.6 us; 4 x 120 -> 40 @ 56x56,
+// 1.1 GFLOP: 24.4 -> 21.2 us; 2 x 216 -> 160 @ 38x38, 1.8 GFLOP: 24.7 against
+// 29.9 us on the split kernel).  Plans that the caller asked Winograd for:
+// at most 32 tiles and 256 or more channels (one image of 512@7 or 256@14).
+// Not when a Winograd variant is forced (NHIP_WINOGRAD_VARIANT);
 // NHIP_WINO_TWIN=0 switches the route off.
 static bool twin_selected(const nhip_conv_plan* p, int n, int oh, int ow) {
-  if (p->igemm_twin == nullptr || variant_requested() != 0 || setting_int("NHIP_WINO_TWIN", 1) == 0) return false;
+  if (p->weight_split == nullptr || variant_requested() != 0 || setting_int("NHIP_WINO_TWIN", 1) == 0) return false;
+  if (p->wino_auto) return 18.0 * n * oh * ow * p->g.k * p->g.c <= 1.5e9;
   return (int64_t)n * ceil_div(oh, 4) * ceil_div(ow, 4) <= 32;
 }
 
 uint64_t conv_winograd_f32_workspace(const nhip_conv_plan* p, int n, int oh, int ow) {
-  if (twin_selected(p, n, oh, ow)) return conv_igemm_f32_workspace(p->igemm_twin, n, oh, ow);
+  if (twin_selected(p, n, oh, ow)) return conv_split_workspace(p, n, oh, ow);
   const int th = (int)ceil_div(oh, 4), tw = (int)ceil_div(ow, 4);
   const int64_t t_pad = round_up((int64_t)n * th * tw, 128);
   if (fused_selected(p, n, oh, ow) && wino_xt_selected(p, n, oh + 2 - p->g.pt - p->g.pb, ow + 2 - p->g.pl - p->g.pr, oh, ow))
@@ -328,7 +333,7 @@ int launch_conv_winograd_f32(const nhip_conv_plan* p, const float* in,
   if (variant_requested() == 0 && kq_supported(p, n, h, w, oh, ow))
     return launch_conv_kq(p, in, residual, out, n, h, w, oh, ow, s);
   if (twin_selected(p, n, oh, ow))
-    return launch_conv_igemm_f32(p->igemm_twin, in, residual, out, n, h, w, oh, ow, ws, ws_bytes, s);
+    return launch_conv_split(p, in, residual, out, n, h, w, oh, ow, ws, ws_bytes, s);
   const bool fused = fused_selected(p, n, oh, ow);
   if (fused && wino_xt_selected(p, n, h, w, oh, ow))
     return launch_wino_gemm_xt(p, in, residual, out, n, h, w, oh, ow, s);

@@ -1,0 +1,137 @@
+"""fp32 Convolution on the split-operand implicit GEMM (every fp32 value as
+three bf16 pieces) against the CPU oracle and against 64-bit sums: the edges
+of its blocks (32 channels, 32 pixels, 8 and 16 input channels, ragged
+reductions), each of its work splits, and non-finite values.
+
+Bound against 64 bits: a sum of n products whose pieces drop terms below
+2^-25 |x w| and whose accumulators round once per 16 products (unit 2^-24):
+2^-25 + 2^-24 (n / 16 + 6 + parts) of sum |x w|, far above what is seen and
+far below the fp32 chain's n 2^-24 for the long reductions here."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import nhip  # noqa: E402
+from oracle import refcpu  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    nhip.init(0)
+
+
+CASES = [
+    # (n, c, h, w, k, kernel, stride, dilation, pad(t,b,l,r), residual, act)
+    (1, 1, 1, 1, 1, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), False, 0),
+    (2, 3, 19, 23, 33, (7, 7), (2, 2), (1, 1), (3, 3, 3, 3), True, 1),     # table order, pixels across images
+    (3, 16, 9, 7, 65, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), False, 1),     # whole 16-channel steps
+    (1, 21, 12, 10, 31, (3, 3), (1, 2), (2, 1), (2, 2, 1, 0), True, 0),    # ragged octet, dilation
+    (2, 24, 8, 8, 64, (5, 5), (2, 2), (1, 1), (2, 2, 2, 2), True, 4),      # whole octets, sigmoid
+    (1, 9, 11, 13, 5, (2, 3), (1, 1), (1, 1), (0, 1, 2, 0), False, 0),     # channels padded by more than a third
+    (1, 600, 4, 5, 40, (1, 1), (2, 2), (1, 1), (0, 0, 0, 0), True, 1),
+    (1, 130, 6, 6, 20, (5, 5), (3, 3), (1, 1), (2, 2, 2, 2), False, 0),    # reduction in several launches' parts
+    (5, 48, 21, 21, 130, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, 1),
+]
+CFGS = [None, "1,1,4,1", "1,2,3,2", "1,4,1,1", "2,1,8,3", "2,4,2,1", "1,1,16,5"]
+
+
+def run(case, x, wt, b, res):
+    n, c, h, w, k, ker, st, dl, pad, _, act = case
+    d = nhip.conv_desc(c, k, ker, st, dl, pad, bias=True, act=act, algorithm=nhip.ALGO_IMPLICIT_GEMM)
+    plan = nhip.Conv2dF32(d, wt, b)
+    nhip.timer_start("conv_split_f32")
+    got = plan.forward(torch.from_numpy(x).cuda(), residual=None if res is None else torch.from_numpy(res).cuda())
+    launches = nhip.timer_stop()[0]
+    return got.cpu().numpy(), launches
+
+
+def data(case, seed):
+    n, c, h, w, k, ker, st, dl, pad, with_res, _ = case
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt = (rng.standard_normal((k, c) + ker) * 0.3).astype(np.float32)
+    oh = (h + pad[0] + pad[1] - dl[0] * (ker[0] - 1) - 1) // st[0] + 1
+    ow = (w + pad[2] + pad[3] - dl[1] * (ker[1] - 1) - 1) // st[1] + 1
+    res = rng.standard_normal((n, k, oh, ow)).astype(np.float32) if with_res else None
+    return x, wt, rng.standard_normal(k).astype(np.float32), res
+
+
+def sums64(case, x, wt):
+    """(sum x w, sum |x w|) per output, in 64 bits."""
+    n, c, h, w, k, ker, st, dl, pad, _, _ = case
+    x = np.pad(x.astype(np.float64), ((0, 0), (0, 0), pad[:2], pad[2:]))
+    oh = (x.shape[2] - dl[0] * (ker[0] - 1) - 1) // st[0] + 1
+    ow = (x.shape[3] - dl[1] * (ker[1] - 1) - 1) // st[1] + 1
+    s, m = np.zeros((n, k, oh, ow)), np.zeros((n, k, oh, ow))
+    for i in range(ker[0]):
+        for j in range(ker[1]):
+            win = x[:, :, i * dl[0]:i * dl[0] + (oh - 1) * st[0] + 1:st[0],
+                    j * dl[1]:j * dl[1] + (ow - 1) * st[1] + 1:st[1]]
+            s += np.einsum("kc,nchw->nkhw", wt[:, :, i, j].astype(np.float64), win)
+            m += np.einsum("kc,nchw->nkhw", np.abs(wt[:, :, i, j]).astype(np.float64), np.abs(win))
+    return s, m
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:5])) + f"k{c[5][0]}s{c[6][0]}")
+@pytest.mark.parametrize("cfg", CFGS)
+def test_conv_split_against_64_bits(case, cfg, nhip_env):
+    for name in ("NHIP_POINTWISE", "NHIP_CONV_KQ", "NHIP_GEMM_DMA", "NHIP_CONV_SMALLK"):
+        nhip_env.setenv(name, "0")
+    if cfg:
+        nhip_env.setenv("NHIP_SPLIT_CFG", cfg)
+    x, wt, b, res = data(case, [CASES.index(case), 5])
+    got, launches = run(case, x, wt, b, res)
+    assert launches == 1
+    s, m = sums64(case, x, wt)
+    exp = s + b.astype(np.float64)[None, :, None, None] + (0 if res is None else res.astype(np.float64))
+    act = case[-1]
+    if act == 1:
+        exp = np.maximum(exp, 0)
+    if act == 4:
+        exp = 1 / (1 + np.exp(-exp))
+    terms = wt[0].size
+    bound = m * (2.0 ** -25 + 2.0 ** -24 * (terms / 16 + 6 + 16)) + 2.0 ** -22 * (np.abs(exp) + 4)
+    assert np.all(np.abs(got - exp) <= bound)
+
+
+@pytest.mark.parametrize("case", [CASES[1], CASES[2], CASES[3], CASES[7]], ids=lambda c: "x".join(map(str, c[:5])))
+def test_conv_split_non_finite_values(case, nhip_env):
+    """Infinities, NaN and values beyond bf16's range of rounding give what a
+    plain fp32 sum gives, and touch no other output."""
+    nhip_env.setenv("NHIP_CONV_KQ", "0")
+    case = case[:-2] + (False, 0)
+    x, wt, b, _ = data(case, 77)
+    flat = x.reshape(-1)
+    at = np.random.default_rng(1).choice(flat.size, 4, replace=False)
+    flat[at] = [np.inf, -np.inf, np.nan, 3.4e38]
+    wt.reshape(-1)[::7] = 0.0  # 0 * inf
+    got, _ = run(case, x, wt, b, None)
+    n, c, h, w, k, ker, st, dl, pad, _, _ = case
+    with np.errstate(all="ignore"):
+        exp = refcpu.conv2d_f32(refcpu.geom(n, c, h, w, k, ker, st, dl, pad), x, wt, b)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(exp))
+    np.testing.assert_array_equal(got[np.isinf(exp)], exp[np.isinf(exp)])
+    fin = np.isfinite(exp)
+    np.testing.assert_allclose(got[fin], exp[fin], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("k", [33, 48, 64])
+@pytest.mark.parametrize("n,c,h,w,ker", [(2, 3, 17, 23, 3), (3, 2, 9, 8, 4), (1, 1, 40, 31, 5)])
+def test_short_reduction_two_channel_blocks(n, c, h, w, ker, k, nhip_env):
+    """The short-reduction kernel's second block of 32 output channels: 33 to
+    64 channels, ragged pixel blocks, residual."""
+    nhip_env.setenv("NHIP_CONV_SMALLK", "2")
+    case = (n, c, h, w, k, (ker, ker), (2, 2), (1, 1), (1, 1, 1, 1), True, 1)
+    x, wt, b, res = data(case, [n, c, k])
+    d = nhip.conv_desc(c, k, (ker, ker), (2, 2), act=1, algorithm=nhip.ALGO_IMPLICIT_GEMM)
+    nhip.timer_start("conv_smallk")
+    got = nhip.Conv2dF32(d, wt, b).forward(torch.from_numpy(x).cuda(), residual=torch.from_numpy(res).cuda())
+    assert nhip.timer_stop()[0] == 1
+    s, m = sums64(case, x, wt)
+    exp = np.maximum(s + b[None, :, None, None].astype(np.float64) + res, 0)
+    bound = m * 2.0 ** -24 * (wt[0].size + 2) + 2.0 ** -22 * (np.abs(exp) + 4)  # an fp32 chain of the products
+    assert np.all(np.abs(got.cpu().numpy() - exp) <= bound)
