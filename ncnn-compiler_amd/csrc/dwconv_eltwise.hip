@@ -77,70 +77,6 @@ __global__ __launch_bounds__(256) void dwconv_f32_kernel(DwArgs a) {
   }
 }
 
-// Same 3x3 stride-1 case with the window unrolled and each thread producing
-// four consecutive outputs of a row (one 3x6 LDS window).
-__global__ __launch_bounds__(256) void dwconv3x3s1_f32_kernel(DwArgs a) {
-  extern __shared__ float lds[];
-  const int band = blockIdx.x % a.bands;
-  const int pgrp = blockIdx.x / a.bands;
-  const int plane0 = pgrp * a.ppb;
-  const int oy0 = band * a.ob;
-  const int iy0 = oy0 - a.pt;
-  const int ix0 = -a.pl;
-  const int per_plane = a.ir * a.lw;
-  const int total_in = a.ppb * per_plane;
-  for (int e = threadIdx.x; e < total_in; e += blockDim.x) {
-    const int pi = e / per_plane;
-    const int r = e - pi * per_plane;
-    const int ry = r / a.lw, rx = r - (r / a.lw) * a.lw;
-    const int plane = plane0 + pi;
-    const int y = iy0 + ry, x = ix0 + rx;
-    float v = 0.f;
-    if (plane < a.planes && (unsigned)y < (unsigned)a.H && (unsigned)x < (unsigned)a.W)
-      v = a.x[(int64_t)plane * a.H * a.W + (int64_t)y * a.W + x];
-    lds[e] = v;
-  }
-  __syncthreads();
-  const int rows = min(a.ob, a.OH - oy0);
-  const int quads = (a.OW + 3) / 4;
-  const int per_out = rows * quads;
-  const int total_out = a.ppb * per_out;
-  for (int e = threadIdx.x; e < total_out; e += blockDim.x) {
-    const int pi = e / per_out;
-    const int r = e - pi * per_out;
-    const int oy = r / quads, ox = (r - (r / quads) * quads) * 4;
-    const int plane = plane0 + pi;
-    if (plane >= a.planes) break;
-    const int c = plane % a.C;
-    const float* wc = a.w + (int64_t)c * 9;
-    float wr[9];
-#pragma unroll
-    for (int t = 0; t < 9; ++t) wr[t] = wc[t];
-    const float* src = lds + pi * per_plane + oy * a.lw + ox;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      float row[6];
-#pragma unroll
-      for (int t = 0; t < 6; ++t) row[t] = (ox + t < a.lw) ? src[i * a.lw + t] : 0.f;
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) acc[q] += row[q + j] * wr[i * 3 + j];
-    }
-    const float b = a.bias[c];
-    float* dst = a.y + (int64_t)plane * a.OH * a.OW + (int64_t)(oy0 + oy) * a.OW + ox;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (ox + q < a.OW) {
-        float v = acc[q] + b;
-        if (a.act == NHIP_ACT_RELU) v = v < 0.f ? 0.f : v;
-        dst[q] = v;
-      }
-    }
-  }
-}
-
 // 3x3 depthwise, stride S (1 or 2), dilation 1, straight from global memory:
 // thread = 4 consecutive outputs of R rows of one plane.  Its input window
 // ((R-1)*S+3 rows x 3S+3 columns) comes in through raw buffer loads, the zero
@@ -853,6 +789,18 @@ int launch_dwconv_f32(const nhip_conv_plan* p, const float* in, float* out,
   // NHIP_DW_PLANES=0 switches it off (tuning and tests), =2 takes it for
   // vector-aligned rows too.
   const int planes_mode = setting_int("NHIP_DW_PLANES", 1);
+  // Column runs from LDS (dw_f32.hip): 5x5; 3x3 at stride 1 whose rows are not
+  // vectors and whose planes the streamed kernel does not take, or takes but
+  // with fewer than 64 pixels (batch 32: 960@7 7.8 -> 6.2 us; 384@14 8.1 on the
+  // streamed kernel against 8.6; 16 x 24 @ 94x94 16.2 -> 11.3); and tensors past
+  // the window kernel's 32-bit offsets.  Rows of vectors are faster on the
+  // window kernel (32 x 144 @ 56x56 28.0 against 31.8 us), stride 2 too (24 x 16
+  // @ 96x96 5.3 against 7.3).  NHIP_DW_RUNS=0 never, =2 wherever it can.
+  const int runs_mode = setting_int("NHIP_DW_RUNS", 1);
+  const bool streamed = k3 && !vec && planes_mode != 0 && hw <= kDwPlaneMax && ow <= kDwRowMax;
+  const bool runs = a.kh == 5 || x_bytes >= (1ull << 31) || (a.sh == 1 && !vec && (!streamed || hw < 64));
+  if ((runs || runs_mode == 2) && planes_mode != 2 && dw_f32_runs_supported(p, n, oh, ow))
+    return launch_dw_f32_runs(p, in, out, n, h, w, oh, ow, s);
   if (k3 && (!vec || planes_mode == 2) && planes_mode != 0 && hw <= kDwPlaneMax && ow <= kDwRowMax &&
       x_bytes < (1ull << 31) && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
     // at most one output row per lane and 16 KB of input per chunk, ppb *
@@ -902,11 +850,6 @@ int launch_dwconv_f32(const nhip_conv_plan* p, const float* in, float* out,
   NHIP_TRY(dw_bands(a.planes, oh, ow, a.kh, a.kw, a.sh, a.dh, a.sw, a.dw, 4, &a.ppb, &a.ob, &a.ir, &a.lw, &a.bands,
                     &lds));
   const int64_t blocks = ceil_div(a.planes, a.ppb) * a.bands;
-  const bool fast = a.kh == 3 && a.kw == 3 && a.sh == 1 && a.sw == 1 && a.dh == 1 && a.dw == 1;
-  if (fast) {
-    NHIP_LAUNCH("dwconv3x3s1_f32", dwconv3x3s1_f32_kernel, dim3((unsigned)blocks), dim3(256), (size_t)lds, s, a);
-    return check_launch("dwconv3x3s1_f32");
-  }
   NHIP_LAUNCH("dwconv_f32", dwconv_f32_kernel, dim3((unsigned)blocks), dim3(256), (size_t)lds, s, a);
   return check_launch("dwconv_f32");
 }

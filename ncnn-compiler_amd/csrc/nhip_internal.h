@@ -291,6 +291,11 @@ int launch_dwconv_f32(const nhip_conv_plan* p, const float* in, float* out,
 int launch_dwconv_int8(const nhip_conv_plan* p, const void* in, int in_is_i8,
                        void* out, int n, int h, int w, int oh, int ow,
                        hipStream_t s);
+// dw_f32.hip: fp32 depthwise 3x3 and 5x5, stride 1 or 2, rows of any width: a
+// column run of outputs per thread from planes in LDS.
+bool dw_f32_runs_supported(const nhip_conv_plan* p, int n, int oh, int ow);
+int launch_dw_f32_runs(const nhip_conv_plan* p, const float* in, float* out, int n, int h, int w, int oh, int ow,
+                       hipStream_t s);
 // dw_int8.hip: int8 depthwise 3x3 and 5x5, stride 1 or 2, 4 x 4 outputs per
 // thread on dot4.
 std::vector<int32_t> dw_int8_pack(const nhip_conv_plan* p, const int8_t* wq);
