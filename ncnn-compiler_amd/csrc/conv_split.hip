@@ -313,7 +313,8 @@ struct SplitCfg {
 // 32-row waves, four or (few workgroups, 32+ steps) eight parts, and long
 // reductions in parts over the launch up to two workgroups per CU (512 ->
 // 512, 3x3 stride 2, one 14x14 image, 288 steps: 28 us in one launch part,
-// 15 in four; 128 -> 256 at 28x28, 72 steps: 10.7 and 9.2).
+// 15 in four; 128 -> 256 at 28x28, 72 steps: 10.7 and 9.2; 1x1, one 7x7
+// image, 960 -> 160, 60 steps, 10 workgroups, weights not in L2: 9.1 and 7.3).
 SplitCfg split_config(const nhip_conv_plan* p, int64_t npix) {
   const int64_t cus = cu_count();
   auto wgs = [&](int tm, int wn) { return ceil_div(npix, 32 * wn) * ceil_div(p->g.k, 32 * tm); };
@@ -328,7 +329,9 @@ SplitCfg split_config(const nhip_conv_plan* p, int64_t npix) {
   } else if (2 * wgs(1, 4) >= 3 * cus) {
     c = {1, 4, 1, 1};
   } else {
-    if (nk >= 64)
+    if (nk >= 32 && nk < 64 && 8 * wgs(1, 1) <= cus)
+      c.splits = 4;
+    else if (nk >= 64)
       while (c.splits < 8 && nk / (8 * c.splits) >= 4 && wgs(1, 1) * c.splits <= 2 * cus) c.splits *= 2;
     if (c.splits == 1 && nk >= 32 && 4 * wgs(1, 1) <= cus) c.kparts = 8;
   }
