@@ -20,8 +20,10 @@
 // transposes the weights to (NCNNToTosa.cpp:1168-1176) — from an NHWC int8
 // image with channels padded to 16.  The register-weight kernel builds that
 // layout for its own input window in LDS, quantizing fp32 input on the way
-// (NHIP_INT8_FUSED_QUANT=0 turns this off); the other kernels read a scratch
-// image that a separate pass quantizes (one pass over HBM).
+// (NHIP_INT8_FUSED_QUANT=0 turns this off), and so does the window kernel of
+// conv_int8_win.hip, which takes most layers; the gather kernel, for layers
+// whose window does not fit there, reads a scratch image that a separate pass
+// quantizes (one pass over HBM).
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -83,11 +85,10 @@ struct Int8Args {
   float os;
   int term, act;
   void* out;           // int8 or fp32 NCHW
-  // footprint kernel only
+  // register-weight kernel only
   int OH, R;           // output rows per workgroup
   int FH, FW, FS;      // input footprint rows / columns / LDS bytes per pixel
   int fp_bytes;        // LDS bytes of the footprint (multiple of 16)
-  int rb_off;             // LDS byte offset of the footprint kernel's reciprocals and biases
   FastDiv cpp_div, fw_div;  // footprint copy: 16-byte channel chunks per pixel, window width
   // register-weight kernel only
   uint32_t out_bytes;     // size of out (< 2^31)
@@ -301,198 +302,6 @@ __global__ __launch_bounds__(kThreads) void conv_int8_kernel(Int8Args g) {
   }
 }
 
-// Footprint variant.  A workgroup owns R whole output rows of one image (at
-// most 128 pixels, padded to 128 MFMA columns) and BM output channels.  The
-// input rows those outputs read (a (R-1)*sh+(kh-1)*dh+1 by
-// (OW-1)*sw+(kw-1)*dw+1 window of the NHWC int8 scratch image, zero halo) are
-// copied into LDS once, with coalesced 16-byte loads; every tap's B fragment
-// is then read straight from that window, so only the weights stream through
-// the two-stage K pipeline (they are shared by all workgroups and stay in
-// L2).  Same MFMA mapping, accumulation and epilogue as conv_int8_kernel.
-template <int BM, int BK>
-__global__ __launch_bounds__(kThreads) void conv_int8_fp_kernel(Int8Args g) {
-  constexpr int BN = 128;
-  constexpr int TM = BM / 64, TN = BN / 64;
-  constexpr int ROW = BK + 16;
-  constexpr int CH = BK / 16;
-  constexpr int A_LD = BM * CH / kThreads;
-  constexpr int ES = BN + 16;
-  extern __shared__ __attribute__((aligned(16))) int8_t dsm[];
-  int8_t* foot = dsm;
-  auto As = [&](int buf) { return dsm + g.fp_bytes + buf * BM * ROW; };
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int li = lane & 31, lh = lane >> 5;
-  const int rgs = (g.OH + g.R - 1) / g.R;
-  const int img = blockIdx.x / rgs, oy0 = (blockIdx.x % rgs) * g.R;
-  const int i0 = blockIdx.y * BM;
-  const int npx = min(g.R, g.OH - oy0) * g.OW;  // valid pixels of this workgroup
-
-  struct Stage {
-    v4i a[A_LD];
-  };
-  auto gload = [&](Stage& st, int kt) {
-#pragma unroll
-    for (int u = 0; u < A_LD; ++u) {
-      const int q = tid + u * kThreads;
-      const int row = q / CH, ch = q % CH;
-      st.a[u] = *reinterpret_cast<const v4i*>(g.w + (int64_t)(i0 + row) * g.kred_pad + kt * BK + ch * 16);
-    }
-  };
-  auto lstore = [&](const Stage& st, int buf) {
-#pragma unroll
-    for (int u = 0; u < A_LD; ++u) {
-      const int q = tid + u * kThreads;
-      const int row = q / CH, ch = q % CH;
-      *reinterpret_cast<v4i*>(As(buf) + row * ROW + ch * 16) = st.a[u];
-    }
-  };
-
-  // The first two weight stages, the footprint and this workgroup's
-  // reciprocals and biases are all requested before anything waits, so
-  // their latencies overlap instead of adding up.
-  const int n = g.kred_pad / BK;
-  Stage s0, s1;
-  gload(s0, 0);
-  if (n > 1) gload(s1, 1);
-  float* rb = reinterpret_cast<float*>(dsm + g.rb_off);  // [BM] reciprocals, then [BM] biases
-  if (tid < BM) {
-    rb[tid] = g.recip[i0 + tid];
-    rb[BM + tid] = g.bias[i0 + tid];
-  }
-
-  // ---- footprint -> LDS, eight 16-byte loads in flight per thread
-  {
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(g.x, g.x_bytes);
-    const int cpp = g.c_pad / 16;
-    const int total = g.FH * g.FW * cpp;
-    const int iy_base = oy0 * g.sh - g.pt;
-    for (int base = 0; base < total; base += 8 * kThreads) {
-      v4i v[8];
-      int dst[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int e = base + q * kThreads + tid;
-        const int pix = fdiv(e, g.cpp_div), ch = e - pix * cpp;
-        const int fy = fdiv(pix, g.fw_div), fx = pix - fy * g.FW;
-        const int iy = iy_base + fy, ix = fx - g.pl;
-        const bool in = e < total && (unsigned)iy < (unsigned)g.H && (unsigned)ix < (unsigned)g.W;
-        v[q] = __builtin_bit_cast(
-            v4i, buf_load_b128(rs, in ? (uint32_t)(((img * g.H + iy) * g.W + ix) * g.c_pad + ch * 16) : kBufOOB));
-        dst[q] = e < total ? pix * g.FS + ch * 16 : -1;
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        if (dst[q] >= 0) *reinterpret_cast<v4i*>(foot + dst[q]) = v[q];
-    }
-  }
-
-  // per-lane window origin (bytes) of each of the wave's pixel columns
-  int fbase[TN];
-#pragma unroll
-  for (int b = 0; b < TN; ++b) {
-    const int pc = min(wn * (BN / 2) + b * 32 + li, npx - 1);
-    const int py = pc / g.OW, px = pc - py * g.OW;
-    fbase[b] = (py * g.sh * g.FW + px * g.sw) * g.FS;
-  }
-
-  v16i acc[TM][TN];
-#pragma unroll
-  for (int a = 0; a < TM; ++a)
-#pragma unroll
-    for (int b = 0; b < TN; ++b)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][b][r] = 0;
-
-  auto compute = [&](int buf, int kt) {
-#pragma unroll
-    for (int s = 0; s < BK / 32; ++s) {
-      const int t = g.ktab[kt * CH + s * 2 + lh];  // this lane's 16-byte k chunk
-      int c0 = t >> 16;
-      const int dy = (t >> 8) & 255, dx = t & 255;
-      if (c0 >= g.c_pad) c0 = 0;  // K padding: the weights there are zero
-      const int koff = (dy * g.FW + dx) * g.FS + c0;
-      v4i af[TM], bf[TN];
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-        af[a] = *reinterpret_cast<const v4i*>(As(buf) + (wm * (BM / 2) + a * 32 + li) * ROW + s * 32 + lh * 16);
-#pragma unroll
-      for (int b = 0; b < TN; ++b) bf[b] = *reinterpret_cast<const v4i*>(foot + fbase[b] + koff);
-#pragma unroll
-      for (int a = 0; a < TM; ++a)
-#pragma unroll
-        for (int b = 0; b < TN; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[a], bf[b], acc[a][b], 0, 0, 0);
-    }
-  };
-
-  {
-    lstore(s0, 0);
-    __syncthreads();  // footprint, first A stage, reciprocals and biases visible
-    int i = 0;
-    for (; i + 1 < n; i += 2) {
-      if (i + 2 < n) gload(s0, i + 2);
-      compute(0, i);
-      lstore(s1, 1);
-      __syncthreads();
-      if (i + 3 < n) gload(s1, i + 3);
-      compute(1, i + 1);
-      if (i + 2 < n) lstore(s0, 0);
-      __syncthreads();
-    }
-    if (i < n) compute(0, i);
-  }
-
-  // ---- epilogue (as conv_int8_kernel), staged in LDS over the footprint
-  __syncthreads();
-  const bool q8 = g.term > 100, relu = g.act == NHIP_ACT_RELU;
-  const int qlo = relu ? 0 : -127;  // requantized ReLU: the saturation's lower bound
-  float* tf = reinterpret_cast<float*>(dsm);
-  int8_t* tq = dsm;
-  auto dequant = [&](int a, int b, int r, int il) {
-#pragma clang fp contract(off)
-    float f = (float)acc[a][b][r];
-    f = f * rb[il];
-    return f + rb[BM + il];
-  };
-  if (q8) {
-#pragma unroll
-    NHIP_I8_EPI({
-      tq[il * ES + jl] = quantize_i8(f, g.os, qlo);
-    })
-  } else {
-#pragma unroll
-    NHIP_I8_EPI(tf[il * ES + jl] = (relu && f < 0.0f) ? 0.0f : f)
-  }
-#undef NHIP_I8_EPI
-  __syncthreads();
-  constexpr int RUNS = BN / 16;
-  for (int q = tid; q < BM * RUNS; q += kThreads) {
-    const int il = q / RUNS, jl = (q % RUNS) * 16;
-    const int i = i0 + il;
-    if (i >= g.m || jl >= npx) continue;
-    const int64_t o = ((int64_t)img * g.m + i) * g.OHW + (int64_t)oy0 * g.OW + jl;
-    const bool whole = jl + 16 <= npx && (o & 15) == 0;
-    if (q8) {
-      int8_t* dst = static_cast<int8_t*>(g.out);
-      if (whole) {
-        *reinterpret_cast<v4i*>(dst + o) = *reinterpret_cast<const v4i*>(&tq[il * ES + jl]);
-      } else {
-        for (int e = 0; e < 16 && jl + e < npx; ++e) dst[o + e] = tq[il * ES + jl + e];
-      }
-    } else {
-      float* dst = static_cast<float*>(g.out);
-      if (whole) {
-#pragma unroll
-        for (int e = 0; e < 16; e += 4)
-          *reinterpret_cast<v4f*>(dst + o + e) = *reinterpret_cast<const v4f*>(&tf[il * ES + jl + e]);
-      } else {
-        for (int e = 0; e < 16 && jl + e < npx; ++e) dst[o + e] = tf[il * ES + jl + e];
-      }
-    }
-  }
-}
-
 // Register-weight variant.  Each wave keeps its 32 output channels' whole
 // reduction (KS 32-byte k steps, 16 bytes per lane and step) in registers,
 // loaded once at the start in k order from the fragment-order copy of the
@@ -500,8 +309,8 @@ __global__ __launch_bounds__(kThreads) void conv_int8_fp_kernel(Int8Args g) {
 // weights would touch 32 cache lines), so no weight passes through LDS and
 // the K loop has no barrier: the MFMAs of step s wait only for step s's
 // weights.  The workgroup (4 waves, 128 channels) shares one footprint
-// window of R whole output rows (at most 32*TN pixels) in LDS, as in
-// conv_int8_fp_kernel.  The MFMA operands are swapped against the other
+// window of R whole output rows (at most 32*TN pixels) in LDS: the NHWC rows
+// those outputs read, zero halo included.  The MFMA operands are swapped against the other
 // kernels (A = pixels, B = weights), so the 32x32 result block is
 // D[pixel][channel]: lane (c, h) holds channel c and, in registers 4g..4g+3,
 // the four consecutive pixels 8g+4h .. 8g+4h+3.  The epilogue stores from
@@ -824,16 +633,23 @@ int launch_conv_int8(const nhip_conv_plan* p, const void* in, int in_is_i8,
   g.out_bytes = (uint32_t)std::min<int64_t>(out_bytes, INT32_MAX);
   // Register-weight kernel: a reduction of 36 k steps (1152 bytes: 128
   // channels at 3x3), whole 128-channel blocks and a footprint window of at
-  // most 2048 16-byte chunks.  NHIP_INT8_RW=0 turns it off, =2 takes two
-  // 32-pixel blocks per wave instead of four (tuning and comparison
-  // switches).
+  // most 2048 16-byte chunks, where its launch is one round of the CUs and keeps
+  // at least 0.6 of it busy (pixels of 128 and workgroups of a CU each): 32 x 128
+  // x 28 x 28 fp32 11.8 us against 15.2 from the window kernel, int8 13.5 against
+  // 13.7, 8 x 128 x 56 x 56 14.2 against 18.0.  In two rounds or half idle the
+  // window kernel is ahead (64 images of 28 x 28 21.9 against 21.0, of 14 x 14
+  // 17.4 against 10.4, 8 of 28 x 28 9.0 against 7.6).  NHIP_INT8_RW=0 turns it
+  // off, =1 takes it wherever it can, =2 too with two 32-pixel blocks per wave
+  // instead of four (tuning and comparison switches).
   {
-    const int mode = setting_int("NHIP_INT8_RW", 1);
+    const int mode = setting_int("NHIP_INT8_RW", -1);
     const int tn = mode == 2 ? 2 : 4;
     const int R = ow > 0 ? std::min(32 * tn / ow, oh) : 0;
     constexpr int KS = kRwKred / 32;
     if (mode != 0 && R >= 1 && p->weight_i8_frag != nullptr && p->m_pad % 128 == 0 && p->kred_pad == kRwKred &&
-        out_bytes < INT32_MAX) {
+        out_bytes < INT32_MAX &&
+        (mode > 0 || (n * ceil_div(oh, R) * (p->m_pad / 128) <= cu_count() &&
+                      (int64_t)g.npix * (p->m_pad / 128) * 10 >= (int64_t)cu_count() * 128 * 6))) {
       Int8Args r = g;
       r.w = p->weight_i8_frag;
       r.OH = oh;
@@ -902,71 +718,14 @@ int launch_conv_int8(const nhip_conv_plan* p, const void* in, int in_is_i8,
       }
     }
   }
-  // The other kernels read the NHWC int8 image.
+  // Window kernel: one launch; NHIP_INT8_FOOTPRINT=0 turns it off (comparison switch).
+  if (setting_int("NHIP_INT8_FOOTPRINT", 1) != 0) {
+    bool taken = false;
+    const int st = launch_conv_int8_win(p, in, in_is_i8, out, n, h, w, oh, ow, s, &taken);
+    if (taken) return st;
+  }
+  // The gather kernel reads the NHWC int8 image.
   NHIP_TRY(quantize());
-  // Footprint kernel when a workgroup's input window fits in LDS (whole rows
-  // of at most 128 output pixels); NHIP_INT8_FOOTPRINT=0 turns it off (a
-  // tuning and comparison switch).
-  {
-    const bool allowed = setting_int("NHIP_INT8_FOOTPRINT", 1) != 0;
-    const int R = ow > 0 ? 128 / ow : 0;
-    const int max_dy = (p->g.kh - 1) * p->g.dh, max_dx = (p->g.kw - 1) * p->g.dw;
-    if (allowed && R >= 1 && p->kred_pad % 128 == 0) {
-      g.OH = oh;
-      g.R = std::min(R, oh);
-      g.FH = (g.R - 1) * p->g.sh + max_dy + 1;
-      g.FW = (ow - 1) * p->g.sw + max_dx + 1;
-      g.FS = p->c_pad + 16;
-      g.fp_bytes = (int)round_up((int64_t)g.FH * g.FW * g.FS, 16);
-      g.cpp_div = fast_div((uint32_t)(p->c_pad / 16));
-      g.fw_div = fast_div((uint32_t)g.FW);
-      // 64 output channels per workgroup (a 128-channel block's epilogue
-      // staging alone would take 72 KB and leave one workgroup per CU)
-      const int bm = 64;
-      // K stage: the widest of 384 / 192 / 128 bytes that divides the
-      // reduction (fewer stages: fewer global-load round trips and barriers
-      // per workgroup; 32x128x28x28 -> 128 channels: 3 stages of 384 bytes, 16.3 against 17.2 us
-      // with 128-byte stages); NHIP_INT8_FP_BK overrides (tuning switch,
-      // ignored when invalid).
-      // operands (footprint + two weight stages) or the epilogue's staging,
-      // then bm reciprocals and bm biases past both
-      auto rb_at = [&](int bk) {
-        const int64_t oper = (int64_t)g.fp_bytes + 2LL * bm * (bk + 16);
-        const int64_t epi = (int64_t)bm * (128 + 16) * 4;
-        return round_up(std::max(oper, epi), 16);
-      };
-      auto lds_for = [&](int bk) { return rb_at(bk) + 2LL * bm * 4; };
-      // Eligible when the window fits beside 128-byte stages in 64 KB; wider
-      // stages may take up to 80 KB (still two workgroups per CU).
-      constexpr int64_t kMaxLds = 80 * 1024;
-      int bk = 128;
-      for (int c : {384, 192})
-        if (p->kred_pad % c == 0 && lds_for(c) <= kMaxLds) {
-          bk = c;
-          break;
-        }
-      if (setting("NHIP_INT8_FP_BK")) {
-        const int c = setting_int("NHIP_INT8_FP_BK", 0);
-        if ((c == 128 || c == 192 || c == 384) && p->kred_pad % c == 0 && lds_for(c) <= kMaxLds) bk = c;
-      }
-      const int64_t lds = lds_for(bk);
-      g.rb_off = (int)rb_at(bk);
-      if (lds_for(128) <= 64 * 1024) {
-        const dim3 grid((unsigned)(n * ceil_div(oh, g.R)), (unsigned)(p->m_pad / bm));
-#define NHIP_FP_CASE(BM_, BK_)                                                                                   \
-  if (bm == BM_ && bk == BK_) {                                                                                 \
-    const auto kernel = conv_int8_fp_kernel<BM_, BK_>;                                                          \
-    NHIP_TRY(ensure_dynamic_lds(reinterpret_cast<const void*>(kernel), (int)kMaxLds));                          \
-    NHIP_LAUNCH("conv_int8_fp", kernel, grid, dim3(kThreads), (unsigned)lds, s, g);                              \
-    return check_launch("conv_int8_fp");                                                                        \
-  }
-        NHIP_FP_CASE(64, 128)
-        NHIP_FP_CASE(64, 192)
-        NHIP_FP_CASE(64, 384)
-#undef NHIP_FP_CASE
-      }
-    }
-  }
   // Tile shape: NHIP_INT8_TILE="bm,bn,bk" overrides (tuning switch, ignored
   // when not valid for the plan).
   int bm = p->m_pad % 128 == 0 ? 128 : 64, bn = 64, bk = 128;

@@ -198,11 +198,10 @@ struct nhip_conv_plan {
   // int8: weights int8 [m_pad][kh*kw*c_pad] (k = (kh, kw, c) order),
   // reciprocal r[c] = ws==0 ? 0 : 1/(ws*is), bias, scales.
   int8_t* weight_i8 = nullptr;
-  // The same int8 weights in MFMA fragment order for the register-weight
-  // kernel, [m_pad/32][kred_pad/32][64 lanes][16 bytes]: lane l of k step s
+  // The same int8 weights in MFMA fragment order for the register-weight and
+  // window kernels (inside weight_i8's buffer), [m_pad/32][kred_pad/32][64 lanes][16 bytes]: lane l of k step s
   // of block b holds row 32b + l%32, bytes 32s + 16(l/32) .. +15, so one
-  // wave's load of a k step is 1 KB contiguous.  Only when that kernel can
-  // take the plan (kred_pad == kRwKred, m_pad a multiple of 128).
+  // wave's load of a k step is 1 KB contiguous.
   int8_t* weight_i8_frag = nullptr;
   // int8 depthwise plans of dw_int8.hip: [C][K][ceil(K/4)] words, a row's taps
   // as bytes, zero padded; inside weight_i8's buffer, after the bytes.
@@ -285,6 +284,10 @@ int launch_wino_gemm(const float* U, const float* V, float* M, int m_pad, int c_
 int launch_conv_int8(const nhip_conv_plan* p, const void* in, int in_is_i8,
                      void* out, int n, int h, int w, int oh, int ow, void* ws,
                      uint64_t ws_bytes, hipStream_t s);
+// conv_int8_win.hip: int8 convolutions in one launch, the input window from
+// NCHW into LDS.  *taken is false (and nothing launched) when no window fits.
+int launch_conv_int8_win(const nhip_conv_plan* p, const void* in, int in_is_i8, void* out, int n, int h, int w, int oh,
+                         int ow, hipStream_t s, bool* taken);
 uint64_t conv_int8_workspace(const nhip_conv_plan* p, int n, int h, int w);
 int launch_dwconv_f32(const nhip_conv_plan* p, const float* in, float* out,
                       int n, int h, int w, int oh, int ow, hipStream_t s);

@@ -1,0 +1,73 @@
+"""The int8 convolution's window kernel at the edges of its tiles: rows shorter
+than a fill group, column segments with a ragged last one, stride-1 1x1 layers
+as one row of pixels, one-row kernels with a stride, channel counts that are no
+multiple of 4, 16 or 32, and every split of a workgroup into channel blocks and
+reduction parts.  Integer sums and separately rounded fp32 steps: bit for bit
+against the oracle, and the same from the gather kernel."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import nhip  # noqa: E402
+from test_gpu_int8 import _gpu, dev, host, oracle, run  # noqa: E402,F401
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # (n, c, h, w, k, kernel, stride, dil, pad, term, act)
+    (2, 5, 6, 3, 33, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 101, 1),      # rows of 3 pixels
+    (1, 7, 5, 1, 1, (3, 1), (1, 1), (1, 1), (1, 1, 0, 0), 1, 0),         # rows of 1 pixel, one channel
+    (2, 3, 9, 150, 32, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), 101, 0),    # 75 columns, three input channels
+    (1, 18, 5, 261, 40, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 102, 1),   # column segments, last one ragged
+    (1, 18, 5, 261, 40, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 2, 1),
+    (3, 34, 19, 17, 65, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), 101, 1),   # 1x1: 323 pixels as one row
+    (1, 64, 1, 2, 96, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), 1, 1),       # 1x1: two pixels
+    (2, 48, 13, 11, 70, (1, 1), (2, 2), (1, 1), (0, 0, 0, 0), 101, 0),   # 1x1 with a stride: every second row
+    (1, 20, 9, 9, 32, (1, 3), (3, 1), (1, 1), (2, 2, 1, 1), 1, 0),       # one-row kernel, padded rows
+    (1, 16, 12, 40, 24, (5, 5), (2, 2), (2, 2), (4, 4, 4, 4), 101, 1),   # dilated, padding wider than a group
+    (1, 600, 14, 12, 32, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 101, 0),  # deep: few pixels per window
+    (1, 1500, 9, 30, 32, (5, 5), (2, 2), (1, 1), (2, 2, 2, 2), 1, 0),    # no window fits: the gather kernel
+]
+CFGS = ["", "1,32,1,1", "1,32,1,8", "2,16,2,2", "1,16,4,1", "3,32,1,4"]
+
+
+def _layer(case, int8_in):
+    n, c, h, w, k, ker, st, dl, pad, term, act = case
+    rng = np.random.default_rng(sum(case[:5]) + term)
+    x = (rng.integers(-128, 128, (n, c, h, w)).astype(np.int8) if int8_in
+         else rng.uniform(-2.5, 2.5, (n, c, h, w)).astype(np.float32))
+    wt = rng.integers(-127, 128, (k, c) + ker).astype(np.int8)
+    scale = rng.uniform(20, 200, k).astype(np.float32)
+    b = rng.normal(0, 0.3, k).astype(np.float32)
+    # an output scale that uses the int8 range
+    spread = 73.0 * 73.0 * np.sqrt(c * ker[0] * ker[1]) / (scale.mean() * 60.0)
+    return nhip.conv_desc(c, k, ker, st, dl, pad, act=act, int8_scale_term=term), x, wt, b, scale, 60.0, 60.0 / spread
+
+
+@pytest.mark.parametrize("int8_in", [True, False], ids=["i8", "f32"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:5])) + f"-t{c[9]}")
+def test_window_kernel_bit_exact(case, int8_in, nhip_env):
+    layer = _layer(case, int8_in)
+    exp = oracle(*layer)
+    for cfg in CFGS:  # a split that does not fit the layer is ignored
+        nhip_env.setenv("NHIP_INT8_WIN_CFG", cfg)
+        np.testing.assert_array_equal(run(*layer), exp, err_msg=f"split {cfg or 'chosen'}")
+    nhip_env.setenv("NHIP_INT8_FOOTPRINT", "0")
+    np.testing.assert_array_equal(run(*layer), exp, err_msg="gather kernel")
+
+
+@pytest.mark.parametrize("int8_in", [True, False], ids=["i8", "f32"])
+def test_unaligned_input_and_output(int8_in):
+    """Tensors at odd element offsets: the kernel's wide loads and stores take any element alignment."""
+    d, x, wt, b, scale, is_, os_ = _layer(CASES[5], int8_in)
+    exp = oracle(d, x, wt, b, scale, is_, os_)
+    conv = nhip.Conv2dInt8(d, wt, b, scale, is_, os_)
+    xd = dev(x)
+    flat = torch.empty(xd.numel() + 1, dtype=xd.dtype, device="cuda")
+    src = flat[1:].view(xd.shape)
+    src.copy_(xd)
+    out = torch.empty(exp.size + 1, dtype=torch.int8, device="cuda")[1:].view(exp.shape)
+    out.fill_(77)
+    conv.forward(src, out=out)
+    np.testing.assert_array_equal(host(out), exp)
