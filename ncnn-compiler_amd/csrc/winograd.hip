@@ -292,17 +292,24 @@ int winograd_prepack_weights(nhip_conv_plan* p, const float* weight) {
 // Launches that leave the Winograd kernels for the split implicit GEMM
 // (conv_split.hip).  The Winograd path costs 12 us (three launches) to 20 us
 // at the least, whatever its size, and its GEMM pads the tiles to 128; the
-// split kernel takes 6 us plus about 10 us per GFLOP of the direct
-// convolution.  Plans whose algorithm the library chose: up to 1.5 GFLOP
-// (9 x 40 -> 24 @ 21x21, 0.07 GFLOP: 19.8 -> 6.6 us; 4 x 120 -> 40 @ 56x56,
-// 1.1 GFLOP: 24.4 -> 21.2 us; 2 x 216 -> 160 @ 38x38, 1.8 GFLOP: 24.7 against
-// 29.9 us on the split kernel).  Plans that the caller asked Winograd for:
-// at most 32 tiles and 256 or more channels (one image of 512@7 or 256@14).
+// split kernel takes 6 us plus 10 to 20 us per GFLOP of the direct convolution.
+// Plans whose algorithm the library chose: up to 0.8 GFLOP (9 x 40 -> 24 @
+// 21x21, 0.07 GFLOP: 19.8 -> 6.6 us; 29 x 80 -> 40 @ 21x21, 0.74: 25.6 -> 17.9; 20
+// x 32 -> 72 @ 30x30, 0.75: 20.8 -> 20.4; but 10 x 32 -> 72 @ 45x45, 0.84: 21.9
+// against 24.7 us on the split kernel, 17 x 32 -> 200 @ 24x24, 1.13: 15.9
+// against 21.4), up to 1.25 with 176 or more input channels (long reductions: 4
+// x 200 -> 136 @ 25x25 24.3 -> 21.8 us), up to 1 with 64 or more and at most 48
+// output channels (23 x 80 -> 40 @ 26x26 25.3 -> 16.8; but 21 x 80 -> 40 @ 30x30,
+// 1.09: 22.5 against 23.8).  Plans that the caller asked Winograd for: at most
+// 32 tiles and 256 or more channels (one image of 512@7 or 256@14).
 // Not when a Winograd variant is forced (NHIP_WINOGRAD_VARIANT);
 // NHIP_WINO_TWIN=0 switches the route off.
 static bool twin_selected(const nhip_conv_plan* p, int n, int oh, int ow) {
   if (p->weight_split == nullptr || variant_requested() != 0 || setting_int("NHIP_WINO_TWIN", 1) == 0) return false;
-  if (p->wino_auto) return 18.0 * n * oh * ow * p->g.k * p->g.c <= 1.5e9;
+  if (p->wino_auto) {
+    const double gflop = 18e-9 * n * oh * ow * p->g.k * p->g.c;
+    return gflop <= 0.8 || (gflop <= 1.25 && p->g.c >= 176) || (gflop <= 1.0 && p->g.c >= 64 && p->g.k <= 48);
+  }
   return (int64_t)n * ceil_div(oh, 4) * ceil_div(ow, 4) <= 32;
 }
 
