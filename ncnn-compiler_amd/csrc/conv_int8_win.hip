@@ -12,7 +12,9 @@
 // weights through LDS with a barrier per stage.  Here
 //   - a workgroup owns R output rows, whole or CW columns of them, of one image
 //     (at most 128 pixels; a stride-1 1x1 layer's image is one row) and MBW
-//     blocks of 32 output channels; an item of its fill is four channels by four pixels: four
+//     blocks of 32 output channels (of 1x1 planes, an InnerProduct's rows: the
+//     images are the pixels of one row, channels contiguous on both sides; 335 x
+//     2081 -> 1783 84.6 us with an image per workgroup, 18.9 us so); an item of its fill is four channels by four pixels: four
 //     loads, a 4 x 4 byte transpose (or sixteen quantizations), four LDS words;
 //   - a wave holds one channel block and one of KP parts of the reduction, its
 //     weights four steps ahead in registers (the first requested before the
@@ -51,12 +53,13 @@ struct WinArgs {
   int steps, kred;     // steps of 32 bytes; reduction bytes (kh, kw, c_pad)
   int mblocks;         // 32-channel blocks of the layer
   int mbw, kp;         // channel blocks and reduction parts of a workgroup
-  int R, CW;           // output rows and columns of a workgroup (CW a multiple of 16 where CW < OW)
+  int R, CW;           // output rows and columns of a workgroup (CW a multiple of 16 where CW < OW, but any for vecs)
   int rgs, segs;       // row groups of an image, column segments of a row
   int FH, FW, FS;      // window rows, columns, bytes per pixel
   int rstep, wsh;      // input rows per window row; window rows per output row
   int xg;              // groups of four columns in a window row's fill
   int tab;             // LDS byte offset of the chunk offsets
+  int vecs;            // 1x1 planes (an InnerProduct): the images are the pixels of one row, channels contiguous
   FastDiv xg_div, c4_div, rg_div, seg_div;
 };
 
@@ -100,7 +103,39 @@ __global__ __launch_bounds__(512, 4) void conv_int8_win_kernel(WinArgs g) {
     }
   }
   __syncthreads();
-  {
+  if (g.vecs) {
+    // items: sixteen channels of one pixel
+    const int groups = g.c_pad >> 4, items = ncol * groups;
+    for (int i = tid; i < items; i += nt) {
+      const int px = i / groups, c0 = 16 * (i - px * groups);
+      const int64_t e = (int64_t)(ox0 + px) * g.C + c0;
+      v4i v = {0, 0, 0, 0};
+      if constexpr (IN8) {
+        const int8_t* src = static_cast<const int8_t*>(g.x) + e;
+        if (c0 + 16 <= g.C) {
+          __builtin_memcpy(&v, src, 16);
+        } else {
+#pragma unroll
+          for (int u = 0; u < 16; ++u)
+            if (c0 + u < g.C) v[u >> 2] |= (int)((uint32_t)(uint8_t)src[u] << (8 * (u & 3)));
+        }
+      } else {
+        const float* src = static_cast<const float*>(g.x) + e;
+        v4f f[4];
+        if (c0 + 16 <= g.C) {
+          __builtin_memcpy(f, src, 64);
+        } else {
+#pragma unroll
+          for (int u = 0; u < 16; ++u) f[u >> 2][u & 3] = c0 + u < g.C ? src[u] : 0.0f;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          v[q] = (int)pack_i8x4(quantize_q(f[q][0], g.is), quantize_q(f[q][1], g.is), quantize_q(f[q][2], g.is),
+                                quantize_q(f[q][3], g.is));
+      }
+      *reinterpret_cast<v4i*>(dsm + px * g.FS + c0) = v;
+    }
+  } else {
     // items: window row, four channels, four pixels (x fastest).  Groups past
     // a row's end start at W - 4 and the last channel group repeats the last
     // channel (the weights of the padding channels are zero).
@@ -225,7 +260,7 @@ __global__ __launch_bounds__(512, 4) void conv_int8_win_kernel(WinArgs g) {
     at = (int64_t)py * g.OW + px;
     return py < nrow ? ncol - px : 0;
   };
-  if (g.kp == 1) {
+  if (g.kp == 1 && !g.vecs) {
     if constexpr (OUT8) {
       __syncthreads();  // (every wave is past its reads of the window)
       if (!live) return;
@@ -313,8 +348,21 @@ __global__ __launch_bounds__(512, 4) void conv_int8_win_kernel(WinArgs g) {
     }
   }
   __syncthreads();
-  // ---- epilogue: four pixels of a channel per thread, TN * 8 threads per channel
   const int rows = g.mbw * 32;
+  if (g.vecs) {  // channels fastest, one result per thread
+    for (int q = tid; q < rows * ncol; q += nt) {
+      const int px = q / rows, row = q - px * rows, ch = blockIdx.y * rows + row;
+      if (ch >= g.M) continue;
+      const float f = rescale(sums[row * TS + px], g.recip[ch], g.bias[ch]);
+      const int64_t o = (int64_t)(ox0 + px) * g.M + ch;
+      if constexpr (OUT8)
+        static_cast<int8_t*>(g.out)[o] = (int8_t)quantize_q(f, g.os, g.qlo);
+      else
+        static_cast<float*>(g.out)[o] = g.relu && f < 0.0f ? 0.0f : f;
+    }
+    return;
+  }
+  // ---- epilogue: four pixels of a channel per thread, TN * 8 threads per channel
   for (int q = tid; q < rows * TN * 8; q += nt) {
     const int row = q / (TN * 8), p = (q - row * TN * 8) * 4, ch = blockIdx.y * rows + row;
     int64_t at;
@@ -365,18 +413,21 @@ int launch_tn(const WinArgs& a, dim3 grid, dim3 block, int lds, bool in8, bool o
 }
 
 struct WinCfg {
-  int h, w, oh, ow;  // the image as the kernel sees it
+  int n, h, w, oh, ow;  // the images as the kernel sees them
+  bool vecs;            // n images of one pixel as one row
   int R, CW, mbw, kp, tn, FH, FW, FS, rstep, wsh, tab, lds;  // R 0: no window fits
 };
 
 WinCfg win_config(const nhip_conv_plan* p, int in_is_i8, int n, int h, int w, int oh, int ow) {
   const ConvGeom& g = p->g;
-  WinCfg c{h, w, oh, ow};
+  WinCfg c{n, h, w, oh, ow};
   // a 1x1 layer with stride 1 and no padding: one row of h * w pixels
   if (g.kh == 1 && g.kw == 1 && g.sh == 1 && g.sw == 1 && oh == h && ow == w && g.pt == 0 && g.pl == 0 &&
       (int64_t)h * w < (1 << 30)) {
-    c.w = c.ow = h * w;
+    c.vecs = h * w == 1;
+    c.w = c.ow = c.vecs ? n : h * w;
     c.h = c.oh = 1;
+    if (c.vecs) c.n = 1;
   }
   const int mblocks = (int)ceil_div(g.k, 32), steps = p->kred_pad / 32;
   c.FS = p->c_pad + 16;
@@ -393,7 +444,7 @@ WinCfg win_config(const nhip_conv_plan* p, int in_is_i8, int n, int h, int w, in
   };
   auto lds_of = [&](int R, int CW, int mbw, int kp) {
     const int t = tn(R, CW) * 32;
-    return std::max(window(R, CW) + 8 * steps, mbw * 32 * (kp > 1 ? (t + 4) * 4 : t + 16));
+    return std::max(window(R, CW) + 8 * steps, mbw * 32 * (kp > 1 || c.vecs ? (t + 4) * 4 : t + 16));
   };
   // Tile, channel blocks and parts with the least estimated clocks on a CU: the
   // larger of what its workgroups keep busy together (fill items, matrix
@@ -410,7 +461,7 @@ WinCfg win_config(const nhip_conv_plan* p, int in_is_i8, int n, int h, int w, in
   auto consider = [&](int r, int cw) {
     const int win = window(r, cw);
     if (r < 1 || win + 8 * steps > kMaxLds) return;
-    const int t = tn(r, cw), tiles = n * (int)ceil_div(c.oh, r) * (int)ceil_div(c.ow, cw);
+    const int t = tn(r, cw), tiles = c.n * (int)ceil_div(c.oh, r) * (int)ceil_div(c.ow, cw);
     const int items = fh(r) * ((std::min(c.w, fw(cw)) + 3) / 4) * ((g.c + 3) / 4);
     int m = 1;
     for (bool last = false; !last; m = std::min(2 * m, mblocks)) {
@@ -426,7 +477,7 @@ WinCfg win_config(const nhip_conv_plan* p, int in_is_i8, int n, int h, int w, in
         const float chain = rounds * (4100.0f + 2700.0f * ((items + nt - 1) / nt) +
                                       (float)steps / k * 157.0f * std::max(1.0f, 0.5f * t));
         float cost = std::max(busy, chain) + 0.5f * std::min(busy, chain);
-        if (cw < c.ow && cw < 64) cost *= 1.05f;  // shorter runs to store
+        if (cw < c.ow && cw < 64 && !c.vecs) cost *= 1.05f;  // shorter runs to store
         if (R == 0 || cost < best) {
           best = cost;
           R = r;
@@ -450,6 +501,9 @@ WinCfg win_config(const nhip_conv_plan* p, int in_is_i8, int n, int h, int w, in
     if (r > 1) consider((r + 1) / 2, cw);
   }
   if (R == 0 && c.ow > 16) consider(1, 16);
+  if (c.vecs)  // (any width: no runs along a row)
+    for (int cw : {16, 8, 4})
+      if (cw < c.ow) consider(1, cw);
   if (R == 0) return c;
   if (const char* env = setting("NHIP_INT8_WIN_CFG")) {  // tuning: rows, columns, channel blocks, parts
     int r = 0, w4 = 0, m = 0, k = 0;
@@ -521,11 +575,12 @@ int launch_conv_int8_win(const nhip_conv_plan* p, const void* in, int in_is_i8, 
   a.wsh = c.wsh;
   a.xg = (int)ceil_div(std::min(c.w, c.FW), 4);
   a.tab = c.tab;
+  a.vecs = c.vecs;
   a.xg_div = fast_div((uint32_t)a.xg);
   a.c4_div = fast_div((uint32_t)ceil_div(a.C, 4));
   a.rg_div = fast_div((uint32_t)a.rgs);
   a.seg_div = fast_div((uint32_t)a.segs);
-  const dim3 grid((unsigned)(n * a.rgs * a.segs), (unsigned)ceil_div(a.mblocks, c.mbw)), block(64 * c.mbw * c.kp);
+  const dim3 grid((unsigned)(c.n * a.rgs * a.segs), (unsigned)ceil_div(a.mblocks, c.mbw)), block(64 * c.mbw * c.kp);
   const bool in8 = in_is_i8 != 0, out8 = p->scale_term > 100;
   if (c.tn == 1) return launch_tn<1>(a, grid, block, c.lds, in8, out8, s);
   if (c.tn == 2) return launch_tn<2>(a, grid, block, c.lds, in8, out8, s);

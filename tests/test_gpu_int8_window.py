@@ -1,6 +1,6 @@
 """The int8 convolution's window kernel at the edges of its tiles: rows shorter
 than a fill group, column segments with a ragged last one, stride-1 1x1 layers
-as one row of pixels, one-row kernels with a stride, channel counts that are no
+and 1x1 planes as one row of pixels, one-row kernels with a stride, channel counts that are no
 multiple of 4, 16 or 32, and every split of a workgroup into channel blocks and
 reduction parts.  Integer sums and separately rounded fp32 steps: bit for bit
 against the oracle, and the same from the gather kernel."""
@@ -23,6 +23,10 @@ CASES = [
     (1, 18, 5, 261, 40, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 2, 1),
     (3, 34, 19, 17, 65, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), 101, 1),   # 1x1: 323 pixels as one row
     (1, 64, 1, 2, 96, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), 1, 1),       # 1x1: two pixels
+    # 1x1 planes: the images as one row of pixels, 16-channel groups with a remainder
+    (133, 50, 1, 1, 70, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), 1, 1),
+    (37, 64, 1, 1, 33, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), 101, 0),
+    (1, 9, 1, 1, 5, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), 102, 1),
     (2, 48, 13, 11, 70, (1, 1), (2, 2), (1, 1), (0, 0, 0, 0), 101, 0),   # 1x1 with a stride: every second row
     (1, 20, 9, 9, 32, (1, 3), (3, 1), (1, 1), (2, 2, 1, 1), 1, 0),       # one-row kernel, padded rows
     (1, 16, 12, 40, 24, (5, 5), (2, 2), (2, 2), (4, 4, 4, 4), 101, 1),   # dilated, padding wider than a group
