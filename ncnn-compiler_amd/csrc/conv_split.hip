@@ -412,8 +412,11 @@ __global__ void conv_splitk_reduce(const float* __restrict__ part, int splits, i
 
 }  // namespace
 
-// The weights [K][C][kh][kw] split into bf16 pieces, in fragment order, and
-// after them (keep_f32: plans that hold them in no other form) as they are.
+// One buffer: the weights [K][C][kh][kw] split into bf16 pieces, in fragment
+// order; (keep_f32: plans that hold them in no other form) as they are; and the
+// table of taps where the reduction runs in (c, kh, kw) order.  Nothing that the
+// kernel reads belongs to another part of the plan: a Winograd plan has no table
+// of its own.
 int conv_split_prepack(nhip_conv_plan* p, const float* weight, bool keep_f32) {
   const int K = p->g.k, C = p->g.c, khw = p->g.kh * p->g.kw;
   const int c8 = (int)round_up(C, 8);
@@ -423,7 +426,8 @@ int conv_split_prepack(nhip_conv_plan* p, const float* weight, bool keep_f32) {
   p->split_nk = (int)ceil_div(p->split_taps ? (int64_t)c8 * khw : (int64_t)C * khw, 16);
   const int nk = p->split_nk;
   const size_t frag = kFrag / 2, pieces = (size_t)(p->m_pad / 32) * nk * kPieces * frag;
-  std::vector<uint16_t> out(pieces + (keep_f32 ? (size_t)2 * K * C * khw : 0), 0);
+  const size_t table = pieces + (keep_f32 ? (size_t)2 * K * C * khw : 0);  // 16-bit words ahead of it
+  std::vector<uint16_t> out(table + (p->split_taps ? 0 : (size_t)2 * nk * 16), 0);
   for (int i = 0; i < K; ++i) {
     const float* wi = weight + (size_t)i * C * khw;
     uint16_t* row = out.data() + (size_t)(i / 32) * nk * kPieces * frag + (size_t)(i % 32) * 8;
@@ -439,10 +443,19 @@ int conv_split_prepack(nhip_conv_plan* p, const float* weight, bool keep_f32) {
     }
   }
   if (keep_f32) std::memcpy(out.data() + pieces, weight, (size_t)K * C * khw * 4);
+  if (!p->split_taps) {
+    std::vector<int32_t> kt((size_t)nk * 16, 0x7fff << 16);
+    for (int k = 0; k < C * khw; ++k) {
+      const int c = k / khw, r = k % khw;
+      kt[k] = (c << 16) | ((r / p->g.kw * p->g.dh) << 8) | (r % p->g.kw * p->g.dw);
+    }
+    std::memcpy(out.data() + table, kt.data(), kt.size() * 4);
+  }
   NHIP_TRY(check_hip(hipMalloc(&p->weight_split, out.size() * 2), "hipMalloc(split conv weight)"));
   NHIP_TRY(check_hip(hipMemcpy(p->weight_split, out.data(), out.size() * 2, hipMemcpyHostToDevice),
                      "hipMemcpy(split conv weight)"));
   p->split_f32 = keep_f32 ? reinterpret_cast<float*>(p->weight_split + pieces) : p->weight;
+  p->split_ktab = p->split_taps ? nullptr : reinterpret_cast<int32_t*>(p->weight_split + table);
   p->split_ldw = keep_f32 ? C * khw : p->kred_pad;
   return ok();
 }
@@ -477,8 +490,8 @@ int launch_conv_split(const nhip_conv_plan* p, const float* in, const float* res
   g.pl = p->g.pl;
   g.dh = p->g.dh;
   g.dw = p->g.dw;
-  g.ktab = p->ktab;
-  g.kred = p->kred;
+  g.ktab = p->split_ktab;
+  g.kred = p->g.c * g.khw;
   g.ohw_div = fast_div((uint32_t)g.OHW);
   g.ow_div = fast_div((uint32_t)g.OW);
   g.oct_div = fast_div((uint32_t)std::max(1, p->g.c % 16 == 0 ? g.c_pad / 16 : g.c_pad / 8));

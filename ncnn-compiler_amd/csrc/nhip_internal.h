@@ -188,6 +188,9 @@ struct nhip_conv_plan {
   // leave the Winograd kernels.
   uint16_t* weight_split = nullptr;
   const float* split_f32 = nullptr;
+  // (inside weight_split's buffer) the taps in (c, kh, kw) order, as in ktab,
+  // where split_taps is 0
+  const int32_t* split_ktab = nullptr;
   int32_t split_nk = 0, split_c_pad = 0, split_taps = 0, split_ldw = 0;
   int32_t wino_auto = 0;      // Winograd chosen by the library, not by the caller
   float* bias = nullptr;      // [m_pad] zero-filled past k (always present)

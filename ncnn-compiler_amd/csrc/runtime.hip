@@ -572,7 +572,7 @@ int nhip_conv2d_f32_create(const nhip_conv_desc* d, const float* weight, const f
         std::copy(weight + (size_t)k * p->kred, weight + (size_t)(k + 1) * p->kred, wp.begin() + (size_t)k * p->kred_pad);
       st = upload(&p->weight, wp, "hipMalloc(conv weight)");
     }
-    if (st == NHIP_STATUS_SUCCESS && (smallk || 3 * round_up(C, 8) > 4 * C)) {  // read in (c, kh, kw) order
+    if (st == NHIP_STATUS_SUCCESS && smallk) {  // the short-reduction kernel's taps
       std::vector<int32_t> kt((size_t)p->kred_pad, 0x7fff << 16);
       for (int k = 0; k < p->kred; ++k) {
         const int c = k / khw, r = k % khw, kh = r / d->kernel_w, kw = r % d->kernel_w;

@@ -135,3 +135,30 @@ def test_short_reduction_two_channel_blocks(n, c, h, w, ker, k, nhip_env):
     exp = np.maximum(s + b[None, :, None, None].astype(np.float64) + res, 0)
     bound = m * 2.0 ** -24 * (wt[0].size + 2) + 2.0 ** -22 * (np.abs(exp) + 4)  # an fp32 chain of the products
     assert np.all(np.abs(got.cpu().numpy() - exp) <= bound)
+
+
+# 3x3 stride-1 layers whose algorithm the library chooses: (n, c, h, w, k, taken by
+# the split kernel).  17 input channels: padding them to eight adds over a third, so
+# the reduction runs by the table of taps.
+AUTO_CASES = [(2, 16, 9, 7, 40, True), (1, 17, 11, 13, 33, True), (3, 17, 8, 8, 16, True), (2, 18, 10, 6, 16, True),
+              (1, 20, 12, 12, 48, True), (1, 33, 7, 9, 35, True), (1, 200, 6, 5, 130, True)]
+
+
+def auto_layer(n, c, h, w, k, seed):
+    rng = np.random.default_rng([n, c, h, w, k, seed])
+    x = rng.standard_normal((n, c, h, w)).astype(np.float32)
+    wt = (rng.standard_normal((k, c, 3, 3)) * 0.3).astype(np.float32)
+    b, res = rng.standard_normal(k).astype(np.float32), rng.standard_normal((n, k, h, w)).astype(np.float32)
+    return x, wt, b, res, nhip.Conv2dF32(nhip.conv_desc(c, k, act=1), wt, b)
+
+
+@pytest.mark.parametrize("n,c,h,w,k,taken", AUTO_CASES)
+def test_chosen_algorithm_against_64_bits(n, c, h, w, k, taken):
+    x, wt, b, res, plan = auto_layer(n, c, h, w, k, 3)
+    nhip.timer_start("conv_split_f32")
+    got = plan.forward(torch.from_numpy(x).cuda(), residual=torch.from_numpy(res).cuda()).cpu().numpy()
+    assert nhip.timer_stop()[0] == (1 if taken else 0)
+    s, m = sums64((n, c, h, w, k, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, 1), x, wt)
+    exp = np.maximum(s + b.astype(np.float64)[None, :, None, None] + res, 0)
+    bound = m * (2.0 ** -25 + 2.0 ** -24 * (wt[0].size / 16 + 6 + 16)) + 2.0 ** -22 * (np.abs(exp) + 4)
+    assert np.all(np.abs(got - exp) <= bound)
