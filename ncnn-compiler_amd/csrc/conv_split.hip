@@ -199,7 +199,10 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
       const uint32_t off = in ? (uint32_t)at * 4u : kBufOOB;
 #pragma unroll
       for (int u = 0; u < 8; ++u) {  // channels past the last one (the weights are zero there) read zero
-        const int soff = __builtin_amdgcn_readfirstlane((ORDER == kTaps ? c0 + u : u) * plane * 4);
+        // (the scalar offset stays inside the tensor, also where it has fewer
+        // than eight channels in all: the range check subtracts it from the size)
+        const int soff =
+            __builtin_amdgcn_readfirstlane((ORDER == kTaps ? c0 + u : ORDER == kTapsRagged && u >= g.C ? 0 : u) * plane * 4);
         st.b[u] = __builtin_bit_cast(
             float, __builtin_amdgcn_raw_buffer_load_b32(xr, ORDER == kTaps || c0 + u < g.C ? off : kBufOOB, soff, 0));
       }

@@ -162,3 +162,16 @@ def test_chosen_algorithm_against_64_bits(n, c, h, w, k, taken):
     exp = np.maximum(s + b.astype(np.float64)[None, :, None, None] + res, 0)
     bound = m * (2.0 ** -25 + 2.0 ** -24 * (wt[0].size / 16 + 6 + 16)) + 2.0 ** -22 * (np.abs(exp) + 4)
     assert np.all(np.abs(got - exp) <= bound)
+
+
+@pytest.mark.parametrize("c", [1, 5, 6, 7, 8, 9])
+def test_fewer_channels_than_an_octet(c, nhip_env):
+    """One image of 6 channels: eight channel planes are more than the whole tensor."""
+    nhip_env.setenv("NHIP_CONV_SMALLK", "0")
+    case = (1, c, 37, 41, 34, (5, 5), (2, 2), (1, 1), (2, 2, 2, 2), False, 0)
+    x, wt, b, _ = data(case, [c, 9])
+    got, launches = run(case, x, wt, b, None)
+    assert launches == 1
+    s, m = sums64(case, x, wt)
+    bound = m * (2.0 ** -25 + 2.0 ** -24 * (wt[0].size / 16 + 6 + 16)) + 2.0 ** -22 * (np.abs(s) + 4)
+    assert np.all(np.abs(got - (s + b.astype(np.float64)[None, :, None, None])) <= bound)
