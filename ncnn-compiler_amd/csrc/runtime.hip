@@ -397,10 +397,14 @@ int check_forward(const nhip_conv_plan* p, const void* in, const void* out, int 
 // Kernels address their input as one raw buffer resource with 32-bit byte
 // offsets, so a launch must keep every tensor below 2^31 bytes.  Larger
 // batches run as consecutive sub-batches of whole images on the same stream.
+int subbatch_images(int64_t max_image_bytes) {
+  const int64_t lim = (int64_t)1 << 31;
+  return (int)std::max<int64_t>(1, (lim - 1) / std::max<int64_t>(max_image_bytes, 1));
+}
+
 template <typename F>
 int for_each_subbatch(int n, int64_t max_image_bytes, F&& run) {
-  const int64_t lim = (int64_t)1 << 31;
-  const int per = (int)std::max<int64_t>(1, (lim - 1) / std::max<int64_t>(max_image_bytes, 1));
+  const int per = subbatch_images(max_image_bytes);
   for (int i0 = 0; i0 < n; i0 += per) NHIP_TRY(run(i0, std::min(per, n - i0)));
   return ok();
 }
@@ -605,10 +609,17 @@ int nhip_conv2d_workspace_size(nhip_conv_t p, int32_t n, int32_t h, int32_t w, u
   if (n < 0 || h <= 0 || w <= 0) return fail(NHIP_STATUS_INVALID_SHAPE, "workspace_size: invalid extent");
   NHIP_TRY(conv_out(p->g, h, w, &oh, &ow));
   switch (p->kind) {
-    case PlanKind::ConvF32:
-      *bytes = p->algorithm == NHIP_CONV_ALGO_WINOGRAD ? conv_winograd_f32_workspace(p, n, oh, ow)
-                                                       : conv_igemm_f32_workspace(p, n, oh, ow);
+    case PlanKind::ConvF32: {
+      auto need = [&](int nb) {
+        return p->algorithm == NHIP_CONV_ALGO_WINOGRAD ? conv_winograd_f32_workspace(p, nb, oh, ow)
+                                                       : conv_igemm_f32_workspace(p, nb, oh, ow);
+      };
+      *bytes = need(n);
+      // a batch that runs in sub-batches: a small one may need more than a large
+      const int per = subbatch_images(4 * std::max((int64_t)p->g.c * h * w, (int64_t)p->g.k * oh * ow));
+      if (n > per) *bytes = std::max({*bytes, need(per), n % per ? need(n % per) : 0});
       break;
+    }
     case PlanKind::ConvInt8:
       *bytes = conv_int8_workspace(p, n, h, w);
       break;

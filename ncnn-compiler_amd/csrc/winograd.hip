@@ -330,7 +330,8 @@ int launch_conv_winograd_f32(const nhip_conv_plan* p, const float* in,
                              int w, int oh, int ow, void* ws, uint64_t ws_bytes,
                              hipStream_t s) {
   const WinoShape ws_ = wino_shape(p, n, h, w, oh, ow);
-  const uint64_t need = conv_winograd_f32_workspace(p, n, oh, ow);
+  const bool twin = twin_selected(p, n, oh, ow);  // (runs with any workspace)
+  const uint64_t need = twin ? 0 : conv_winograd_f32_workspace(p, n, oh, ow);
   if (need > 0 && (ws == nullptr || ws_bytes < need))
     return fail(NHIP_STATUS_OUTPUT_CAPACITY_INSUFFICIENT,
                 "winograd conv: workspace of " + std::to_string(need) + " bytes required");
@@ -339,7 +340,7 @@ int launch_conv_winograd_f32(const nhip_conv_plan* p, const float* in,
   // forced with NHIP_WINOGRAD_VARIANT)
   if (variant_requested() == 0 && kq_supported(p, n, h, w, oh, ow))
     return launch_conv_kq(p, in, residual, out, n, h, w, oh, ow, s);
-  if (twin_selected(p, n, oh, ow))
+  if (twin)
     return launch_conv_split(p, in, residual, out, n, h, w, oh, ow, ws, ws_bytes, s);
   const bool fused = fused_selected(p, n, oh, ow);
   if (fused && wino_xt_selected(p, n, h, w, oh, ow))

@@ -175,3 +175,35 @@ def test_fewer_channels_than_an_octet(c, nhip_env):
     s, m = sums64(case, x, wt)
     bound = m * (2.0 ** -25 + 2.0 ** -24 * (wt[0].size / 16 + 6 + 16)) + 2.0 ** -22 * (np.abs(s) + 4)
     assert np.all(np.abs(got - (s + b.astype(np.float64)[None, :, None, None])) <= bound)
+
+
+def test_remainder_of_sub_batches_has_its_workspace():
+    """A batch past 2 GiB runs in sub-batches of whole images: 2674 of these and
+    one more, which alone splits its reduction over the launch."""
+    c, k, hw, n = 1024, 64, 14, 2675
+    rng = np.random.default_rng(31)
+    wt = (rng.standard_normal((k, c, 1, 1)) * 0.05).astype(np.float32)
+    plan = nhip.Conv2dF32(nhip.conv_desc(c, k, (1, 1), pad=(0, 0, 0, 0)), wt, rng.standard_normal(k).astype(np.float32))
+    assert plan.workspace_size(1, hw, hw) > 0
+    x = torch.randn((n, c, hw, hw), device="cuda")
+    got = plan.forward(x)
+    assert torch.equal(got[-1:], plan.forward(x[-1:].clone()))
+    assert torch.equal(got[:2], plan.forward(x[:2674])[:2])
+
+
+@pytest.mark.parametrize("n,large,c,k,hw,ker", [(8, 32, 1024, 64, 14, 1), (1, 4, 128, 32, 52, 3)])
+def test_workspace_of_a_larger_batch(n, large, c, k, hw, ker):
+    """A launch whose parts do not fit the workspace that the largest batch needs runs in one part."""
+    rng = np.random.default_rng(32)
+    wt, b = (rng.standard_normal((k, c, ker, ker)) * 0.05).astype(np.float32), rng.standard_normal(k).astype(np.float32)
+    plan = nhip.Conv2dF32(nhip.conv_desc(c, k, (ker, ker), pad=(ker // 2,) * 4), wt, b)
+    x = torch.randn((n, c, hw, hw), device="cuda")
+    need = plan.workspace_size(n, hw, hw)
+    assert need > 0
+    ref = torch.nn.functional.conv2d(x.cpu().double(), torch.from_numpy(wt).double(), torch.from_numpy(b).double(),
+                                     padding=ker // 2)
+    for size in {0, need - 1, min(need, plan.workspace_size(large, hw, hw))}:
+        nhip.timer_start("conv_split_f32")
+        got = plan.forward(x, workspace=torch.empty(size, dtype=torch.uint8, device="cuda"))
+        assert nhip.timer_stop()[0] == 1
+        assert ((got.cpu().double() - ref).norm() / ref.norm()).item() < 1e-6
