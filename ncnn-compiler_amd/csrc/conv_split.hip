@@ -12,10 +12,13 @@
 // fp32's own half ulp.  Sums stay in fp32 accumulators, and a matrix
 // instruction adds 16 products before it rounds where the fp32 one adds two.
 //
-// Non-finite values: an infinity or NaN (or a value that rounds to bf16's
-// infinity) turns the pieces below it into NaN, and so every output that it
-// touches; such outputs are recomputed in the epilogue as a plain fp32 sum,
-// so what the caller sees is fp32 arithmetic's infinities and NaNs.
+// Where the pieces do not stand for the number: an infinity or NaN (or a value
+// that rounds to bf16's infinity) turns the pieces below it into NaN, and x0 w0
+// may overflow where x w does not.  A wave whose block is not all finite at the
+// end forms it again on v_mfma_f32_32x32x2_f32, so what the caller sees is fp32
+// arithmetic's infinities and NaNs.  (32 x 64 -> 128 below, 47 us: 96 with every
+// value NaN, 69 with one; 69 on the fp32 kernel that it replaced, 6070 and 2650
+// where each such output was summed by one lane.)
 //
 // GEMM view: D[i][j] = sum_k A[i][k] B[k][j], i an output channel, j an output
 // pixel over the whole batch.  The reduction runs over octets of eight input
@@ -78,8 +81,6 @@ struct SplitArgs {
   const int* ktab;       // (c, kh, kw) order: c << 16 | dy << 8 | dx
   int kred;
   FastDiv ohw_div, ow_div, oct_div, kw_div;  // by OHW, OW, steps (kTaps) or octets per tap, KW
-  const float* wf;       // fp32 weights [m_pad][ldw] in (c, kh, kw) order, for outputs to recompute
-  int ldw;
   float* d;              // out NCHW, or partial sums [split][m][npix]
   const float* bias;
   const float* residual;
@@ -102,30 +103,6 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t (&p)[kPieces])
     a -= __uint_as_float(u << 16);
     b -= __uint_as_float(u & 0xffff0000u);
   }
-}
-
-// Output (i, pixel j) over steps [k_begin, k_end) as a plain fp32 sum.
-template <bool TAPS>
-__device__ float recompute(const SplitArgs& g, int i, int j, int k_begin, int k_end) {
-  const int img = j / g.OHW, rem = j - img * g.OHW, oh = rem / g.OW, ow = rem - oh * g.OW;
-  const float* xi = g.x + (int64_t)img * g.C * g.H * g.W;
-  float acc = 0.f;
-  for (int k = k_begin * 16; k < k_end * 16; ++k) {
-    int c, r;
-    if (TAPS) {
-      r = k / g.c_pad;
-      c = k - r * g.c_pad;
-      if (r >= g.khw || c >= g.C) continue;
-    } else {
-      if (k >= g.kred) break;
-      c = k / g.khw;
-      r = k - c * g.khw;
-    }
-    const int y = oh * g.sh - g.pt + r / g.KW * g.dh, x = ow * g.sw - g.pl + r % g.KW * g.dw;
-    if ((unsigned)y >= (unsigned)g.H || (unsigned)x >= (unsigned)g.W) continue;
-    acc += xi[((int64_t)c * g.H + y) * g.W + x] * g.wf[(int64_t)i * g.ldw + c * g.khw + r];
-  }
-  return acc;
 }
 
 template <int TM, int ORDER>
@@ -233,6 +210,22 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
                                                     0, 0, 0);
       }
   };
+  // The same steps in fp32, into acc: a lane's weights put together again (a sum
+  // of their pieces is exact), value u of its eight the k of one instruction.
+  auto mul32 = [&](const Step& st) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int a = 0; a < TM; ++a) {
+        float w[kPieces];
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p) {
+          const uint32_t two = (uint32_t)st.a[a][p][u >> 1];
+          w[p] = __uint_as_float(u & 1 ? two & 0xffff0000u : two << 16);
+        }
+        acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[0] + w[1] + w[2], st.b[u], acc[a], 0, 0, 0);
+      }
+  };
   {
     Step s0, s1;
     load(s0, k_begin);
@@ -244,13 +237,33 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
       load(s1, k + 3);
     }
   }
+  float chk = 0.f;
+#pragma unroll
+  for (int a = 0; a < TM; ++a)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      acc[a][r] += low[a][r];
+      chk = __builtin_fmaf(acc[a][r], 0.f, chk);  // 0, or NaN from the first one that is not finite
+    }
+  if (__builtin_expect(__ballot(chk != chk) != 0, 0)) {
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][r] = 0.f;
+#pragma unroll 1
+    for (int k = k_begin; k < k_end; ++k) {
+      Step st;
+      load(st, k);
+      mul32(st);
+    }
+  }
   // partial blocks, [kpart][row][pixel] with the row pitch padded
   const int TS = BN + 4;
   float* mine = lds + kpart * BM * TS + wn * 32 + li;
 #pragma unroll
   for (int a = 0; a < TM; ++a)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) mine[(a * 32 + (r & 3) + 8 * (r >> 2) + 4 * lh) * TS] = acc[a][r] + low[a][r];
+    for (int r = 0; r < 16; ++r) mine[(a * 32 + (r & 3) + 8 * (r >> 2) + 4 * lh) * TS] = acc[a][r];
   __syncthreads();
   const int ohw = g.OHW;
   const bool raw = g.splits > 1, vec = (ohw & 3) == 0;
@@ -260,18 +273,6 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
     if (i >= g.m || j >= g.npix) continue;
     v4f v = *reinterpret_cast<const v4f*>(&lds[row * TS + lc]);
     for (int w = 1; w < g.kparts; ++w) v += *reinterpret_cast<const v4f*>(&lds[(w * BM + row) * TS + lc]);
-    if (__builtin_expect(__ballot(v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3]) != 0, 0)) {
-      // a sum that met a non-finite piece: formed again as a plain fp32 sum
-      for (int e = 0; e < 4; ++e) {
-        const float t = e == 0 ? v[0] : e == 1 ? v[1] : e == 2 ? v[2] : v[3];
-        if (t == t || j + e >= g.npix) continue;
-        const float f = recompute<ORDER != kTable>(g, i, j + e, z_begin, z_end);
-        if (e == 0) v[0] = f;
-        if (e == 1) v[1] = f;
-        if (e == 2) v[2] = f;
-        if (e == 3) v[3] = f;
-      }
-    }
     if (raw) {
       float* dst = part + (int64_t)i * g.npix + j;
       if (vec) {
@@ -370,21 +371,29 @@ int launch_tm(const nhip_conv_plan* p, const SplitArgs& g, hipStream_t s) {
 }
 
 // Eight values' pieces, each piece's eight 16-bit words at out[piece * stride]
-// (fixed-length loops without branches: the compiler vectorizes them).
+// (fixed-length loops without branches: the compiler vectorizes them).  Their sum
+// is the value, whatever it is: the first piece of an infinity or NaN is that and
+// the others 0, and a number never rounds up to infinity.
 void split_octet(const float (&x)[8], uint16_t* out, size_t stride) {
   float v[8];
   for (int e = 0; e < 8; ++e) v[e] = x[e];
   for (int q = 0; q < kPieces; ++q) {
-    uint32_t u[8];
+    uint32_t u[8], rest[8];
     std::memcpy(u, v, sizeof(u));
-    for (int e = 0; e < 8; ++e) {  // to nearest even; NaN stays NaN
-      const uint32_t nan = (u[e] & 0x7fffffffu) > 0x7f800000u ? 0xffffffffu : 0u;
-      const uint32_t r = (u[e] + 0x7fffu + ((u[e] >> 16) & 1)) & 0xffff0000u;
-      u[e] = (r & ~nan) | ((u[e] | 0x400000u) & 0xffff0000u & nan);
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t mag = u[e] & 0x7fffffffu;
+      const uint32_t special = mag >= 0x7f800000u ? 0xffffffffu : 0u, nan = mag > 0x7f800000u ? 0x400000u : 0u;
+      const uint32_t up = mag < 0x7f7f8000u ? 0x7fffu + ((u[e] >> 16) & 1) : 0u;  // to nearest even
+      u[e] = (((u[e] + up) & ~special) | ((u[e] | nan) & special)) & 0xffff0000u;
+      rest[e] = ~special;
     }
     float h[8];
     std::memcpy(h, u, sizeof(h));
     for (int e = 0; e < 8; ++e) v[e] -= h[e];
+    std::memcpy(u, v, sizeof(u));
+    for (int e = 0; e < 8; ++e) rest[e] &= u[e];
+    std::memcpy(v, rest, sizeof(v));
+    std::memcpy(u, h, sizeof(u));
     for (int e = 0; e < 8; ++e) out[q * stride + e] = (uint16_t)(u[e] >> 16);
   }
 }
@@ -416,11 +425,10 @@ __global__ void conv_splitk_reduce(const float* __restrict__ part, int splits, i
 }  // namespace
 
 // One buffer: the weights [K][C][kh][kw] split into bf16 pieces, in fragment
-// order; (keep_f32: plans that hold them in no other form) as they are; and the
-// table of taps where the reduction runs in (c, kh, kw) order.  Nothing that the
-// kernel reads belongs to another part of the plan: a Winograd plan has no table
-// of its own.
-int conv_split_prepack(nhip_conv_plan* p, const float* weight, bool keep_f32) {
+// order, and the table of taps where the reduction runs in (c, kh, kw) order.
+// Nothing that the kernel reads belongs to another part of the plan: a Winograd
+// plan has no table of its own.
+int conv_split_prepack(nhip_conv_plan* p, const float* weight) {
   const int K = p->g.k, C = p->g.c, khw = p->g.kh * p->g.kw;
   const int c8 = (int)round_up(C, 8);
   // taps order pads the channels to eight: not where that adds over a third
@@ -429,8 +437,7 @@ int conv_split_prepack(nhip_conv_plan* p, const float* weight, bool keep_f32) {
   p->split_nk = (int)ceil_div(p->split_taps ? (int64_t)c8 * khw : (int64_t)C * khw, 16);
   const int nk = p->split_nk;
   const size_t frag = kFrag / 2, pieces = (size_t)(p->m_pad / 32) * nk * kPieces * frag;
-  const size_t table = pieces + (keep_f32 ? (size_t)2 * K * C * khw : 0);  // 16-bit words ahead of it
-  std::vector<uint16_t> out(table + (p->split_taps ? 0 : (size_t)2 * nk * 16), 0);
+  std::vector<uint16_t> out(pieces + (p->split_taps ? 0 : (size_t)2 * nk * 16), 0);
   for (int i = 0; i < K; ++i) {
     const float* wi = weight + (size_t)i * C * khw;
     uint16_t* row = out.data() + (size_t)(i / 32) * nk * kPieces * frag + (size_t)(i % 32) * 8;
@@ -445,21 +452,18 @@ int conv_split_prepack(nhip_conv_plan* p, const float* weight, bool keep_f32) {
       split_octet(x, row + (size_t)(k / 16) * kPieces * frag + (size_t)(k % 16 / 8) * 256, frag);
     }
   }
-  if (keep_f32) std::memcpy(out.data() + pieces, weight, (size_t)K * C * khw * 4);
   if (!p->split_taps) {
     std::vector<int32_t> kt((size_t)nk * 16, 0x7fff << 16);
     for (int k = 0; k < C * khw; ++k) {
       const int c = k / khw, r = k % khw;
       kt[k] = (c << 16) | ((r / p->g.kw * p->g.dh) << 8) | (r % p->g.kw * p->g.dw);
     }
-    std::memcpy(out.data() + table, kt.data(), kt.size() * 4);
+    std::memcpy(out.data() + pieces, kt.data(), kt.size() * 4);
   }
   NHIP_TRY(check_hip(hipMalloc(&p->weight_split, out.size() * 2), "hipMalloc(split conv weight)"));
   NHIP_TRY(check_hip(hipMemcpy(p->weight_split, out.data(), out.size() * 2, hipMemcpyHostToDevice),
                      "hipMemcpy(split conv weight)"));
-  p->split_f32 = keep_f32 ? reinterpret_cast<float*>(p->weight_split + pieces) : p->weight;
-  p->split_ktab = p->split_taps ? nullptr : reinterpret_cast<int32_t*>(p->weight_split + table);
-  p->split_ldw = keep_f32 ? C * khw : p->kred_pad;
+  p->split_ktab = p->split_taps ? nullptr : reinterpret_cast<int32_t*>(p->weight_split + pieces);
   return ok();
 }
 
@@ -499,8 +503,6 @@ int launch_conv_split(const nhip_conv_plan* p, const float* in, const float* res
   g.ow_div = fast_div((uint32_t)g.OW);
   g.oct_div = fast_div((uint32_t)std::max(1, p->g.c % 16 == 0 ? g.c_pad / 16 : g.c_pad / 8));
   g.kw_div = fast_div((uint32_t)g.KW);
-  g.wf = p->split_f32;
-  g.ldw = p->split_ldw;
   g.d = out;
   g.bias = p->bias;
   g.residual = residual;

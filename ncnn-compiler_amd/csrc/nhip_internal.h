@@ -182,16 +182,13 @@ struct nhip_conv_plan {
   // 3x3 depthwise plans: [C][12], the nine taps, the bias, two zeros.
   float* weight_dw12 = nullptr;
   // The weights split into three bf16 pieces in MFMA fragment order
-  // (conv_split.hip), [m_pad/32][split_nk][3][64 lanes][8], and where the fp32
-  // weights [K][split_ldw] in (c, kh, kw) order are (in the same buffer, or
-  // `weight`): implicit-GEMM plans, and Winograd plans for the launches that
-  // leave the Winograd kernels.
+  // (conv_split.hip), [m_pad/32][split_nk][3][64 lanes][8]: implicit-GEMM plans,
+  // and Winograd plans for the launches that leave the Winograd kernels.
   uint16_t* weight_split = nullptr;
-  const float* split_f32 = nullptr;
-  // (inside weight_split's buffer) the taps in (c, kh, kw) order, as in ktab,
-  // where split_taps is 0
+  // (in the same buffer) the taps in (c, kh, kw) order, as in ktab, where
+  // split_taps is 0
   const int32_t* split_ktab = nullptr;
-  int32_t split_nk = 0, split_c_pad = 0, split_taps = 0, split_ldw = 0;
+  int32_t split_nk = 0, split_c_pad = 0, split_taps = 0;
   int32_t wino_auto = 0;      // Winograd chosen by the library, not by the caller
   float* bias = nullptr;      // [m_pad] zero-filled past k (always present)
   int32_t m_pad = 0, kred = 0, kred_pad = 0, c_pad = 0;
@@ -265,7 +262,7 @@ int launch_dwpw_lds_f32(const nhip_conv_plan* dw, const nhip_conv_plan* pw, cons
                         const float* residual, float* out, int n, int h, int w, int oh, int ow, hipStream_t s);
 // conv_split.hip: implicit GEMM on the bf16 matrix instructions, the fp32
 // operands split exactly into three bf16 pieces (any fp32 convolution).
-int conv_split_prepack(nhip_conv_plan* p, const float* weight, bool keep_f32);
+int conv_split_prepack(nhip_conv_plan* p, const float* weight);
 uint64_t conv_split_workspace(const nhip_conv_plan* p, int n, int oh, int ow);
 int launch_conv_split(const nhip_conv_plan* p, const float* in, const float* residual, float* out, int n, int h,
                       int w, int oh, int ow, void* ws, uint64_t ws_bytes, hipStream_t s);

@@ -562,13 +562,12 @@ int nhip_conv2d_f32_create(const nhip_conv_desc* d, const float* weight, const f
     st = winograd_prepack_weights(p, weight);
     if (st == NHIP_STATUS_SUCCESS) st = conv_kq_prepack(p, weight, C, K, 3, 3);
     p->wino_auto = d->algorithm == NHIP_CONV_ALGO_AUTO;
-    if (st == NHIP_STATUS_SUCCESS && (p->wino_auto || C >= kWinoTwinMinC)) st = conv_split_prepack(p, weight, true);
+    if (st == NHIP_STATUS_SUCCESS && (p->wino_auto || C >= kWinoTwinMinC)) st = conv_split_prepack(p, weight);
   } else {
     const int khw = d->kernel_h * d->kernel_w;
     p->kred = C * khw;
     p->kred_pad = (int)round_up(p->kred, 16);
-    // row-major weights: the 1x1 kernels and the short-reduction one; the
-    // others hold them with the split ones
+    // row-major weights: the 1x1 kernels and the short-reduction one
     const bool smallk = p->kred <= 32 && K <= 64, rows = khw == 1 || smallk;
     if (rows) {
       std::vector<float> wp((size_t)p->m_pad * p->kred_pad, 0.f);
@@ -585,7 +584,7 @@ int nhip_conv2d_f32_create(const nhip_conv_desc* d, const float* weight, const f
       st = upload(&p->ktab, kt, "hipMalloc(conv ktab)");
     }
     if (st == NHIP_STATUS_SUCCESS) st = conv_kq_prepack(p, weight, C, K, d->kernel_h, d->kernel_w);
-    if (st == NHIP_STATUS_SUCCESS) st = conv_split_prepack(p, weight, !rows);
+    if (st == NHIP_STATUS_SUCCESS) st = conv_split_prepack(p, weight);
     if (st == NHIP_STATUS_SUCCESS && khw == 1 && K <= 32) {
       std::vector<float> ck((size_t)C * 32, 0.f);
       for (int k = 0; k < K; ++k)

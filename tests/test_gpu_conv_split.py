@@ -207,3 +207,25 @@ def test_workspace_of_a_larger_batch(n, large, c, k, hw, ker):
         got = plan.forward(x, workspace=torch.empty(size, dtype=torch.uint8, device="cuda"))
         assert nhip.timer_stop()[0] == 1
         assert ((got.cpu().double() - ref).norm() / ref.norm()).item() < 1e-6
+
+
+@pytest.mark.parametrize("cfg", [None, "1,1,1,1", "2,2,2,1", "1,2,3,2"])
+@pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[2], CASES[3]], ids=lambda c: "x".join(map(str, c[:5])))
+def test_products_near_overflow(case, cfg, nhip_env):
+    """x w is finite where the product of their rounded bf16 pieces is not: one product per sum, just below the
+    largest fp32 number."""
+    for name in ("NHIP_POINTWISE", "NHIP_CONV_KQ", "NHIP_GEMM_DMA", "NHIP_CONV_SMALLK"):
+        nhip_env.setenv(name, "0")
+    if cfg:
+        nhip_env.setenv("NHIP_SPLIT_CFG", cfg)
+    case = case[:-2] + (False, 0)
+    x, wt, b, _ = data(case, 5)
+    rng = np.random.default_rng(6)
+    x[:] = 0
+    x.reshape(-1)[x.size // 2] = -1.8428e19
+    wt[:] = rng.uniform(1.8426e19, 1.8428e19, wt.shape) * rng.choice([-1, 1], wt.shape)
+    got, launches = run(case, x, wt, b * 0, None)
+    assert launches == 1
+    s, _ = sums64(case, x, wt)
+    assert np.abs(s).max() > 3.39e38 and np.abs(s).max() < 3.4028e38
+    np.testing.assert_allclose(got, s, rtol=2.0 ** -22)
