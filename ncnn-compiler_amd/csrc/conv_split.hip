@@ -4,21 +4,24 @@
 //
 // v_mfma_f32_32x32x16_bf16 does 16 times the work of v_mfma_f32_32x32x2_f32
 // in a cycle.  x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0),
-// x2 = bf16(x - x0 - x1), each rounded to nearest even, loses nothing: three
-// 8-bit significands cover fp32's 24 bits, the differences are exact in fp32,
-// and bf16 has fp32's exponent range.  Of the nine products of two such sums
+// x2 = bf16(x - x0 - x1), each rounded to nearest even, loses nothing while x2 is
+// a normal number or 0 (|x| from 2^-102 on, or fewer bits): three 8-bit
+// significands cover fp32's 24 bits, the differences are exact in fp32, and bf16
+// has fp32's exponent range.  Of the nine products of two such sums
 // the six of order 2^-16 and above are formed (x0 w0, x0 w1, x1 w0, x0 w2,
 // x1 w1, x2 w0); the three dropped are below 2^-26 of |x w|, a quarter of
 // fp32's own half ulp.  Sums stay in fp32 accumulators, and a matrix
 // instruction adds 16 products before it rounds where the fp32 one adds two.
 //
 // Where the pieces do not stand for the number: an infinity or NaN (or a value
-// that rounds to bf16's infinity) turns the pieces below it into NaN, and x0 w0
-// may overflow where x w does not.  A wave whose block is not all finite at the
-// end forms it again on v_mfma_f32_32x32x2_f32, so what the caller sees is fp32
-// arithmetic's infinities and NaNs.  (32 x 64 -> 128 below, 47 us: 96 with every
-// value NaN, 69 with one; 69 on the fp32 kernel that it replaced, 6070 and 2650
-// where each such output was summed by one lane.)
+// that rounds to bf16's infinity) turns the pieces below it into NaN, x0 w0 may
+// overflow where x w does not, and a last piece below fp32's normal numbers may be
+// rounded (an input of 1e-36 would keep 15 bits).  A wave that met such an input,
+// or whose block holds such a sum or one that is not finite, forms its block again on
+// v_mfma_f32_32x32x2_f32, so what the caller sees is fp32 arithmetic, with its
+// infinities and NaNs.  (32 x 64 -> 128 below, 47 us: 96 with every value NaN, 69
+// with one; 69 on the fp32 kernel that it replaced, 6070 and 2650 where each such
+// output was summed by one lane.)  Weights that small are scaled by the plan.
 //
 // GEMM view: D[i][j] = sum_k A[i][k] B[k][j], i an output channel, j an output
 // pixel over the whole batch.  The reduction runs over octets of eight input
@@ -50,8 +53,10 @@
 // x 32: 107 -> 100.  Error against 64 bits, normwise: 4.3e-7 -> 1.4e-7 (576
 // terms), 2.8e-7 -> 0.95e-7 (3384 terms), 1.5e-7 -> 0.7e-7 (1x1, 232 terms).
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <limits>
 
 #include "nhip_internal.h"
 
@@ -70,6 +75,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 // 16; channels per tap in octets, the last one possibly ragged.
 enum { kTable, kTaps, kTapsRagged };
 
+// 2 |x| - 1 in bits for |x| = 2^-102: below it the last piece may be subnormal.
+constexpr uint32_t kSmall = 25u << 24;
+
 struct SplitArgs {
   const uint16_t* a;     // split weights in fragment order
   int nk, mblocks;       // steps of 16 k, 32-row blocks
@@ -80,6 +88,7 @@ struct SplitArgs {
   int C, c_pad, khw, KW, H, W, OW, OHW, sh, sw, pt, pl, dh, dw;
   const int* ktab;       // (c, kh, kw) order: c << 16 | dy << 8 | dx
   int kred;
+  const float* unscale;  // [m_pad] powers of two that undo the scaling of the weights' rows, or null
   FastDiv ohw_div, ow_div, oct_div, kw_div;  // by OHW, OW, steps (kTaps) or octets per tap, KW
   float* d;              // out NCHW, or partial sums [split][m][npix]
   const float* bias;
@@ -150,6 +159,14 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
     float b[8];
   };
   const char* abase = reinterpret_cast<const char*>(g.a) + (int64_t)(i0 / 32) * g.nk * (kPieces * kFrag) + lane * 16;
+  // the lane's value u of step k, in the table's order
+  auto gather = [&](int k, int u) {
+    const int ka = min(k, g.nk - 1), t0 = g.ktab[ka * 16 + u], t1 = g.ktab[ka * 16 + 8 + u], e = lh ? t1 : t0;
+    const int c = e >> 16, kk = k * 16 + lh * 8 + u;
+    const int y = iy0 + ((e >> 8) & 255), x = ix0 + (e & 255);
+    const bool in = pix_ok && k < k_end && kk < g.kred && (unsigned)y < (unsigned)g.H && (unsigned)x < (unsigned)g.W;
+    return buf_load_f32(xr, in ? (uint32_t)(pbase + (c * g.H + y) * g.W + x) * 4u : kBufOOB);
+  };
   auto load = [&](Step& st, int k) {  // past the end: the input reads zero
     const int ka = min(k, g.nk - 1);
 #pragma unroll
@@ -159,13 +176,7 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
         st.a[a][p] = *reinterpret_cast<const v4i*>(abase + ((int64_t)a * g.nk + ka) * (kPieces * kFrag) + p * kFrag);
     if constexpr (ORDER == kTable) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int t0 = g.ktab[ka * 16 + u], t1 = g.ktab[ka * 16 + 8 + u], e = lh ? t1 : t0;
-        const int c = e >> 16, kk = k * 16 + lh * 8 + u;
-        const int y = iy0 + ((e >> 8) & 255), x = ix0 + (e & 255);
-        const bool in = pix_ok && k < k_end && kk < g.kred && (unsigned)y < (unsigned)g.H && (unsigned)x < (unsigned)g.W;
-        st.b[u] = buf_load_f32(xr, in ? (uint32_t)(pbase + (c * g.H + y) * g.W + x) * 4u : kBufOOB);
-      }
+      for (int u = 0; u < 8; ++u) st.b[u] = gather(k, u);
     } else {
       const int o = ORDER == kTaps ? k : 2 * k + lh, per_tap = ORDER == kTaps ? g.c_pad / 16 : g.c_pad / 8;
       const int tap = fdiv(o, g.oct_div), c0 = (o - tap * per_tap) * (ORDER == kTaps ? 16 : 8);
@@ -192,14 +203,34 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
   for (int a = 0; a < TM; ++a)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[a][r] = low[a][r] = 0.f;
+  // The smallest magnitude met but 0, as 2 |x| - 1 in bits (0: the largest): 1.5
+  // operations a value.  Left to the compiler they wait at the loop's end, sixteen
+  // registers and a wave per SIMD more (up to 11% of a launch), so they are tied
+  // to the values before the split (few registers to spare there) or closed after it.
+  uint32_t least = 0xffffffffu;
+  auto track = [&](float a, float b) {
+    least = min(least, min((__float_as_uint(a) << 1) - 1, (__float_as_uint(b) << 1) - 1));
+  };
   auto mul = [&](const Step& st) {
     uint32_t w[4][kPieces];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) split2(st.b[2 * u], st.b[2 * u + 1], w[u]);
+    for (int u = 0; u < 4; ++u) {
+      float x0 = st.b[2 * u], x1 = st.b[2 * u + 1];
+      if constexpr (ORDER == kTable) {
+        track(x0, x1);
+        asm("" : "+v"(least), "+v"(x0), "+v"(x1));
+      }
+      split2(x0, x1, w[u]);
+    }
     bf16x8 f[kPieces];
 #pragma unroll
     for (int p = 0; p < kPieces; ++p)
       f[p] = __builtin_bit_cast(bf16x8, (v4i{(int)w[0][p], (int)w[1][p], (int)w[2][p], (int)w[3][p]}));
+    if constexpr (ORDER != kTable) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) track(st.b[2 * u], st.b[2 * u + 1]);
+      asm volatile("" : "+v"(least));
+    }
     constexpr int kProd[6][2] = {{0, 0}, {1, 0}, {0, 1}, {1, 1}, {2, 0}, {0, 2}};
 #pragma unroll
     for (int q = 0; q < 6; ++q)
@@ -212,6 +243,9 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
   };
   // The same steps in fp32, into acc: a lane's weights put together again (a sum
   // of their pieces is exact), value u of its eight the k of one instruction.
+  float un[TM];  // what undoes the scaling of the lane's rows
+#pragma unroll
+  for (int a = 0; a < TM; ++a) un[a] = 1.f;
   auto mul32 = [&](const Step& st) {
 #pragma unroll
     for (int u = 0; u < 8; ++u)
@@ -223,7 +257,7 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
           const uint32_t two = (uint32_t)st.a[a][p][u >> 1];
           w[p] = __uint_as_float(u & 1 ? two & 0xffff0000u : two << 16);
         }
-        acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[0] + w[1] + w[2], st.b[u], acc[a], 0, 0, 0);
+        acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32((w[0] + w[1] + w[2]) * un[a], st.b[u], acc[a], 0, 0, 0);
       }
   };
   {
@@ -244,18 +278,42 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
     for (int r = 0; r < 16; ++r) {
       acc[a][r] += low[a][r];
       chk = __builtin_fmaf(acc[a][r], 0.f, chk);  // 0, or NaN from the first one that is not finite
+      if (r & 1) track(acc[a][r - 1], acc[a][r]);  // (sums near the subnormal numbers: two roundings there are more than one)
     }
-  if (__builtin_expect(__ballot(chk != chk) != 0, 0)) {
+  if (__builtin_expect(__ballot(least < kSmall || chk != chk) != 0, 0)) {
+#pragma unroll
+    for (int a = 0; a < TM; ++a) {
+      if (g.unscale) un[a] = g.unscale[i0 + 32 * a + li];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[a][r] = 0.f;
+    }
+#pragma unroll 1
+    for (int k = k_begin; k < k_end; ++k) {
+      if constexpr (ORDER == kTable) {  // one value at a time: eight would take a wave per SIMD's registers
+#pragma unroll 1
+        for (int u = 0; u < 8; ++u) {
+          const float x = gather(k, u);
+#pragma unroll
+          for (int a = 0; a < TM; ++a) {
+            float w = 0.f;
+#pragma unroll
+            for (int p = 0; p < kPieces; ++p)
+              w += __uint_as_float((uint32_t)*reinterpret_cast<const uint16_t*>(
+                       abase + ((int64_t)a * g.nk + k) * (kPieces * kFrag) + p * kFrag + 2 * u) << 16);
+            acc[a] = __builtin_amdgcn_mfma_f32_32x32x2f32(w * un[a], x, acc[a], 0, 0, 0);
+          }
+        }
+      } else {
+        Step st;
+        load(st, k);
+        mul32(st);
+      }
+    }
+  } else if (g.unscale) {
 #pragma unroll
     for (int a = 0; a < TM; ++a)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[a][r] = 0.f;
-#pragma unroll 1
-    for (int k = k_begin; k < k_end; ++k) {
-      Step st;
-      load(st, k);
-      mul32(st);
-    }
+      for (int r = 0; r < 16; ++r) acc[a][r] *= g.unscale[i0 + 32 * a + (r & 3) + 8 * (r >> 2) + 4 * lh];
   }
   // partial blocks, [kpart][row][pixel] with the row pitch padded
   const int TS = BN + 4;
@@ -428,6 +486,11 @@ __global__ void conv_splitk_reduce(const float* __restrict__ part, int splits, i
 // order, and the table of taps where the reduction runs in (c, kh, kw) order.
 // Nothing that the kernel reads belongs to another part of the plan: a Winograd
 // plan has no table of its own.
+//
+// Rows with weights too small for their pieces (below 2^-100, as the channels that
+// training leaves dead have them) are stored times a power of two that lifts the
+// smallest there, as far as the largest stays finite (it does where they span less
+// than 2^226), and their sums are scaled back: [m_pad] factors after the table.
 int conv_split_prepack(nhip_conv_plan* p, const float* weight) {
   const int K = p->g.k, C = p->g.c, khw = p->g.kh * p->g.kw;
   const int c8 = (int)round_up(C, 8);
@@ -436,10 +499,27 @@ int conv_split_prepack(nhip_conv_plan* p, const float* weight) {
   p->split_c_pad = c8;
   p->split_nk = (int)ceil_div(p->split_taps ? (int64_t)c8 * khw : (int64_t)C * khw, 16);
   const int nk = p->split_nk;
+  std::vector<float> unscale;
+  for (int i = 0; i < K; ++i) {
+    float least = std::numeric_limits<float>::max(), most = 0.f;
+    for (size_t j = 0; j < (size_t)C * khw; ++j) {
+      const float mag = std::fabs(weight[(size_t)i * C * khw + j]);
+      if (mag < std::numeric_limits<float>::infinity()) {
+        least = std::min(least, mag > 0.f ? mag : least);
+        most = std::max(most, mag);
+      }
+    }
+    const int up = most > 0.f ? std::min(-100 - std::ilogb(least), 126 - std::ilogb(most)) : 0;
+    if (up <= 0) continue;
+    unscale.resize((size_t)p->m_pad, 1.f);
+    unscale[i] = std::ldexp(1.f, -up);
+  }
   const size_t frag = kFrag / 2, pieces = (size_t)(p->m_pad / 32) * nk * kPieces * frag;
-  std::vector<uint16_t> out(pieces + (p->split_taps ? 0 : (size_t)2 * nk * 16), 0);
+  const size_t factors = pieces + (p->split_taps ? 0 : (size_t)2 * nk * 16);  // 16-bit words ahead of them
+  std::vector<uint16_t> out(factors + 2 * unscale.size(), 0);
   for (int i = 0; i < K; ++i) {
     const float* wi = weight + (size_t)i * C * khw;
+    const float scale = unscale.empty() ? 1.f : 1.f / unscale[i];
     uint16_t* row = out.data() + (size_t)(i / 32) * nk * kPieces * frag + (size_t)(i % 32) * 8;
     for (int k = 0; k < (p->split_taps ? c8 * khw : C * khw); k += 8) {
       float x[8];
@@ -449,6 +529,8 @@ int conv_split_prepack(nhip_conv_plan* p, const float* weight) {
       } else {
         for (int e = 0; e < 8; ++e) x[e] = k + e < C * khw ? wi[k + e] : 0.f;
       }
+      if (scale != 1.f)
+        for (int e = 0; e < 8; ++e) x[e] *= scale;
       split_octet(x, row + (size_t)(k / 16) * kPieces * frag + (size_t)(k % 16 / 8) * 256, frag);
     }
   }
@@ -460,9 +542,11 @@ int conv_split_prepack(nhip_conv_plan* p, const float* weight) {
     }
     std::memcpy(out.data() + pieces, kt.data(), kt.size() * 4);
   }
+  if (!unscale.empty()) std::memcpy(out.data() + factors, unscale.data(), unscale.size() * 4);
   NHIP_TRY(check_hip(hipMalloc(&p->weight_split, out.size() * 2), "hipMalloc(split conv weight)"));
   NHIP_TRY(check_hip(hipMemcpy(p->weight_split, out.data(), out.size() * 2, hipMemcpyHostToDevice),
                      "hipMemcpy(split conv weight)"));
+  p->split_unscale = unscale.empty() ? nullptr : reinterpret_cast<float*>(p->weight_split + factors);
   p->split_ktab = p->split_taps ? nullptr : reinterpret_cast<int32_t*>(p->weight_split + pieces);
   return ok();
 }
@@ -499,6 +583,7 @@ int launch_conv_split(const nhip_conv_plan* p, const float* in, const float* res
   g.dw = p->g.dw;
   g.ktab = p->split_ktab;
   g.kred = p->g.c * g.khw;
+  g.unscale = p->split_unscale;
   g.ohw_div = fast_div((uint32_t)g.OHW);
   g.ow_div = fast_div((uint32_t)g.OW);
   g.oct_div = fast_div((uint32_t)std::max(1, p->g.c % 16 == 0 ? g.c_pad / 16 : g.c_pad / 8));

@@ -188,6 +188,9 @@ struct nhip_conv_plan {
   // (in the same buffer) the taps in (c, kh, kw) order, as in ktab, where
   // split_taps is 0
   const int32_t* split_ktab = nullptr;
+  // (in the same buffer) [m_pad] factors that undo the scaling of rows with
+  // weights too small for bf16 pieces; null where no row is scaled
+  const float* split_unscale = nullptr;
   int32_t split_nk = 0, split_c_pad = 0, split_taps = 0;
   int32_t wino_auto = 0;      // Winograd chosen by the library, not by the caller
   float* bias = nullptr;      // [m_pad] zero-filled past k (always present)

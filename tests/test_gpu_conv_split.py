@@ -229,3 +229,39 @@ def test_products_near_overflow(case, cfg, nhip_env):
     s, _ = sums64(case, x, wt)
     assert np.abs(s).max() > 3.39e38 and np.abs(s).max() < 3.4028e38
     np.testing.assert_allclose(got, s, rtol=2.0 ** -22)
+
+
+@pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[2], CASES[3], CASES[7]], ids=lambda c: "x".join(map(str, c[:5])))
+@pytest.mark.parametrize("what", ["x", "one x", "w", "rows", "both"])
+def test_operands_that_bf16_pieces_do_not_hold(case, what, nhip_env):
+    """Numbers whose lower pieces would fall under bf16's smallest subnormal (2^-133): inputs down to fp32's, one
+    such input among zeros, weights of all rows or of some, and products near the subnormal numbers.  A chain of
+    fp32 sums: n + 2 roundings of 2^-24 of sum |x w|, or of 2^-149 where the sums are subnormal."""
+    for name in ("NHIP_POINTWISE", "NHIP_CONV_KQ", "NHIP_GEMM_DMA", "NHIP_CONV_SMALLK"):
+        nhip_env.setenv(name, "0")
+    case = case[:-2] + (False, 0)
+    x, wt, b, _ = data(case, 15)
+    scales = [1e-33, 1e-36, 3e-38, 1e-41]
+    for scale in scales if what != "rows" else [1]:
+        xs, ws = x, wt
+        if what == "x":
+            xs = x * np.float32(scale)
+        if what == "one x":
+            xs = np.zeros_like(x)
+            xs.reshape(-1)[x.size // 2] = scale * 1.2345678
+        if what == "w":
+            ws = wt * np.float32(scale)
+        if what == "both":
+            xs, ws = x * np.float32(scale * 1e10), wt * np.float32(3e-9)
+        if what == "rows":
+            ws = wt.copy()
+            for i in range(ws.shape[0]):
+                ws[i] *= np.float32([1, 1e-37, 0, 1e-41, 1e30][i % 5])
+                if i % 2:
+                    ws[i].reshape(-1)[::3] *= np.float32(1e-20)
+        xs, ws = xs.astype(np.float32), ws.astype(np.float32)
+        got, launches = run(case, xs, ws, b * 0, None)
+        assert launches == 1
+        s, m = sums64(case, xs, ws)
+        terms = wt[0].size
+        assert np.all(np.abs(got - s) <= m * 2.0 ** -24 * (terms + 2) + 2.0 ** -149 * (terms + 2)), scale
