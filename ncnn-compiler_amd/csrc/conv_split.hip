@@ -9,9 +9,13 @@
 // significands cover fp32's 24 bits, the differences are exact in fp32, and bf16
 // has fp32's exponent range.  Of the nine products of two such sums
 // the six of order 2^-16 and above are formed (x0 w0, x0 w1, x1 w0, x0 w2,
-// x1 w1, x2 w0); the three dropped are below 2^-26 of |x w|, a quarter of
-// fp32's own half ulp.  Sums stay in fp32 accumulators, and a matrix
-// instruction adds 16 products before it rounds where the fp32 one adds two.
+// x1 w1, x2 w0); the three dropped (x1 w2, x2 w1, x2 w2) are below 2^-23 of |x w|
+// (on 40 million random pairs at most 2^-24.1, 2.7% above 2^-26).  Sums stay in
+// fp32 accumulators, and a matrix instruction adds 16 products before it rounds
+// where the fp32 one adds two.  So from two products on a sum is nearer to 64
+// bits than a chain of fp32 (normwise 2.6e-8 against 3.1e-8 at two, 3.1e-8 against
+// 7.4e-8 at 16, emulated); one product alone is not (2.60e-8 against 2.53e-8, up
+// to 1.7 half ulps against one) and is formed in fp32.
 //
 // Where the pieces do not stand for the number: an infinity or NaN (or a value
 // that rounds to bf16's infinity) turns the pieces below it into NaN, x0 w0 may
@@ -46,7 +50,7 @@
 // What bounds it: large launches the operand stream from L2 (a step brings 5
 // or 8 KB for 6 or 12 matrix instructions: 36 steps, 1568 workgroups, 41 us at
 // 64 -> 128 above, 70 us on fp32 matrix instructions and LDS tiles), small ones
-// the chain of load round trips (8 x 16 ... 6 us, the call itself).  Before ->
+// the chain of load round trips (9 x 40 -> 24 at 21x21: 6.6 us).  Before ->
 // now: 3x3 stride 2, 128 -> 256 at 28x28 x 32: 79 -> 41 us; 8 x 64 -> 128 at
 // 56x56: 29 -> 16; 5x5 stride 2, 4 x 256 -> 32 at 103x103: 237 -> 78; 1 x 168 ->
 // 24 at 80x80: 27 -> 14; 1x1, 576 -> 96 at 14x14: 17 -> 7.4; stem 7x7 at 224x224
@@ -80,7 +84,7 @@ constexpr uint32_t kSmall = 25u << 24;
 
 struct SplitArgs {
   const uint16_t* a;     // split weights in fragment order
-  int nk, mblocks;       // steps of 16 k, 32-row blocks
+  int nk;                // steps of 16 k
   int m;                 // output channels
   const float* x;        // input NCHW
   uint32_t x_bytes;      // < 2^31
@@ -207,7 +211,8 @@ __global__ __launch_bounds__(TM == 1 ? 1024 : 512) void conv_split_kernel(SplitA
   // operations a value.  Left to the compiler they wait at the loop's end, sixteen
   // registers and a wave per SIMD more (up to 11% of a launch), so they are tied
   // to the values before the split (few registers to spare there) or closed after it.
-  uint32_t least = 0xffffffffu;
+  // (A sum of one product is formed in fp32 whatever its values.)
+  uint32_t least = g.kred > 1 ? 0xffffffffu : 0u;
   auto track = [&](float a, float b) {
     least = min(least, min((__float_as_uint(a) << 1) - 1, (__float_as_uint(b) << 1) - 1));
   };
@@ -562,7 +567,6 @@ int launch_conv_split(const nhip_conv_plan* p, const float* in, const float* res
   SplitArgs g{};
   g.a = p->weight_split;
   g.nk = p->split_nk;
-  g.mblocks = p->m_pad / 32;
   g.m = p->g.k;
   g.x = in;
   g.x_bytes = (uint32_t)((size_t)n * p->g.c * h * w * sizeof(float));
