@@ -283,6 +283,10 @@ __global__ __launch_bounds__(512, 4) void conv_int8_win_kernel(WinArgs g) {
           *reinterpret_cast<v4i*>(stage + li * RS + b * 32 + 16 * lh) = y;
         }
       }
+      // the rows read back are other lanes' of this wave
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       const int run = lane % kRunsPer, row0 = lane / kRunsPer;
       int64_t p;
       const int left = place(run * 16, p);
