@@ -44,3 +44,25 @@ def test_dw_runs_bit_exact(case, act, nhip_env):
                                   flat[off:].reshape(n, c, h, w), wt, b)
         exp = refcpu.relu_f32(exp) if act else exp
     np.testing.assert_array_equal(got, exp)
+
+
+@pytest.mark.parametrize("n,c,h,w", [(3, 200, 1040, 1040), (2, 300, 1037, 1041)])
+def test_wide_rows_past_32_bit_offsets(n, c, h, w):
+    """Rows that the column runs cannot stage in a tensor past 2 GiB: whole images at a time on the window kernel,
+    bit for bit what it gives on one image's half of the channels."""
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    nhip.init(0)
+    rng = np.random.default_rng([n, c, w])
+    wt, b = rng.standard_normal((c, 1, 3, 3)).astype(np.float32), rng.standard_normal(c).astype(np.float32)
+
+    def plan(lo, hi):
+        return nhip.DwConv2dF32(nhip.conv_desc(hi - lo, hi - lo, act=1, group=hi - lo), wt[lo:hi], b[lo:hi])
+
+    x = torch.randn((n, c, h, w), device="cuda")
+    assert x.numel() * 4 >= 2 ** 31
+    nhip.timer_start("dw3x3s")
+    got = plan(0, c).forward(x)
+    assert nhip.timer_stop()[0] == 2
+    for i in range(n):
+        for lo, hi in ((0, c // 2), (c // 2, c)):
+            assert torch.equal(got[i:i + 1, lo:hi], plan(lo, hi).forward(x[i:i + 1, lo:hi].contiguous()))
