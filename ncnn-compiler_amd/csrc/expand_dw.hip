@@ -485,12 +485,7 @@ int launch_tq(const EdArgs& a, int tq, int n, int strips, int lds, hipStream_t s
 // the 1x1: 26.1 against 33.6 us at 14x14 (64 -> 384 -> 64), 28.4 against
 // 30.2 at 28x28 (32 -> 192 -> 32), 24.2 against 34.3 at 28x28 stride 2; at
 // 56x56 61.1 against 53.6 and at 112x112 77.5 against 67.9 (many strips,
-// each workgroup's phases serial: per-workgroup latency dominates).  Not either
-// where 96 input channels meet planes of 128 or more pixels in so few
-// workgroups that the phases, not the launches, are the time: one or two
-// images of 96 -> 576 at 14x14 take 15 us in the fused kernel, 9 in the two
-// layers' (MobileNetV2 on one 224x224 image 302 -> 283 us over the graph, on
-// two of 191x191 295 -> 279; from three images on, and at 9x9, no gain).
+// each workgroup's phases serial: per-workgroup latency dominates).
 bool pwdw_supported(const nhip_conv_plan* pw, const nhip_conv_plan* dw, int n, int h, int w) {
   if (!pw || !dw || pw->kind != PlanKind::ConvF32 || dw->kind != PlanKind::DwConvF32) return false;
   const int mode = setting_int("NHIP_PWDW", 1);
@@ -513,10 +508,25 @@ bool pwdw_supported(const nhip_conv_plan* pw, const nhip_conv_plan* dw, int n, i
   EdCfg c;
   if (!ed_config(p.c, p.k, h, w, d.sh, &c)) return false;
   const int oh = (h - 1) / d.sh + 1, ow = (w - 1) / d.sw + 1;
-  if (mode != 2 && p.c == 96 && h * w >= 128 && 8 * n * ceil_div(p.k, c.sl) * ceil_div(oh, c.r) <= cu_count())
-    return false;
   return (int64_t)n * p.c * h * w < INT32_MAX && (int64_t)n * p.k * oh * ow < INT32_MAX && n <= 65535 &&
          ceil_div(oh, c.r) <= 65535;
+}
+
+// Whether the fused kernel is also the faster one, for a caller that can run the
+// two layers instead (the graph executor): not where 96 input channels meet
+// planes of 128 or more pixels in so few workgroups that the phases, not the
+// launches, are the time: one or two images of 96 -> 576 at 14x14 take 15 us in
+// the fused kernel, 9 in the two layers' (MobileNetV2 on one 224x224 image 302 ->
+// 283 us over the graph, on two of 191x191 295 -> 279; from three images on, and
+// at 9x9, no gain).  NHIP_PWDW=2: always.
+bool pwdw_preferred(const nhip_conv_plan* pw, const nhip_conv_plan* dw, int n, int h, int w) {
+  n = std::max(1, std::min(n, 65535));
+  if (!pwdw_supported(pw, dw, n, h, w)) return false;
+  if (setting_int("NHIP_PWDW", 1) == 2) return true;
+  EdCfg c;
+  if (!ed_config(pw->g.c, pw->g.k, h, w, dw->g.sh, &c)) return false;
+  const int oh = (h - 1) / dw->g.sh + 1;
+  return !(pw->g.c == 96 && h * w >= 128 && 8 * n * ceil_div(pw->g.k, c.sl) * ceil_div(oh, c.r) <= cu_count());
 }
 
 int launch_pwdw_f32(const nhip_conv_plan* pw, const nhip_conv_plan* dw, const float* in, float* out, int n, int h,

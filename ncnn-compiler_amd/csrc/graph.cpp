@@ -25,6 +25,7 @@ namespace nhip {
 bool kernel_timer_active();
 bool stream_capturing(void* stream);
 int setting_int(const char* name, int fallback);
+bool pwdw_preferred(const nhip_conv_plan* pw, const nhip_conv_plan* dw, int n, int h, int w);
 uint64_t settings_generation();
 int graph_capture_begin(void* stream);
 int graph_capture_end(void* stream, void** exec);
@@ -1369,14 +1370,12 @@ int run_ops(nhip_graph& g, int n, const std::vector<Shape>& sh, const void* cons
     const Op& op = g.ops[oi];
     if (op.kind == OpKind::Input || done[oi]) continue;
     if (op.kind == OpKind::ConvF32 && op.pwdw_dw >= 0) {
-      // expand -> depthwise in one kernel where that kernel takes the pair
-      // (its shape policy says where it is preferred); the depthwise's own
+      // expand -> depthwise in one kernel where that kernel takes the pair and
+      // is preferred; the depthwise's own
       // fusion into the 1x1 after it is then not used
       const Op& d = g.ops[op.pwdw_dw];
       const Shape& a = sh[op.in[0]];
-      int32_t sup = 0;
-      TRY(nhip_conv1x1_dw_f32_supported(op.conv, d.conv, n, (int32_t)a.d[1], (int32_t)a.d[2], &sup));
-      if (sup) {
+      if (nhip::pwdw_preferred(op.conv, d.conv, n, (int32_t)a.d[1], (int32_t)a.d[2])) {
         ptr[d.out] = out_buf(d.out);
         TRY(nhip_conv1x1_dw_f32_forward(op.conv, d.conv, (const float*)ptr[op.in[0]], (float*)ptr[d.out], n,
                                         (int32_t)a.d[1], (int32_t)a.d[2], stream));

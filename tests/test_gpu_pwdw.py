@@ -177,6 +177,16 @@ def test_expand_dw_not_taken_for_unsupported_pairs(nhip_env):
     assert not nhip.conv1x1_dw_supported(pw, dw, 2, 14, 14)
 
 
+@pytest.mark.parametrize("n", [1, 2])
+def test_few_images_are_supported(n):
+    """A pair that the graph executor runs as two layers at these batches is still taken by the call itself."""
+    rng = np.random.default_rng(61)
+    pw, dw = _layers(rng, 96, 576, 1, R, R)
+    assert nhip.conv1x1_dw_supported(pw, dw, n, 14, 14)
+    xd = dev(rng.uniform(-1, 1, (n, 96, 14, 14)).astype(np.float32))
+    assert_close(host(nhip.conv1x1_dw_forward(pw, dw, xd)), host(dw.forward(pw.forward(xd))), RTOL, f"{n} images")
+
+
 def test_expand_dw_random_shapes(nhip_env):
     """40 seeded random pairs (channels, planes of 1-30 rows and columns,
     stride, activations, batch) with every plane the kernel takes: the fused
