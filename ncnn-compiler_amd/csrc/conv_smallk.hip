@@ -212,7 +212,11 @@ void launch_steps(const SmallkArgs& a, int act, dim3 grid, hipStream_t s) {
 // 32-bit buffer offsets; by default only from four 32-pixel blocks per CU
 // (measured on the 224x224 stem: 26.4 against 35.7 us at batch 32, 11.1
 // against 13.1 at batch 8, equal at batch 2, 9.7 against 8.6 us for one
-// image, where the implicit GEMM's smaller tiles spread better).
+// image, where the implicit GEMM's smaller tiles spread better).  With 33 to 64
+// channels, gathered twice and with half the waves each, only reductions of at
+// most 16 from 64 blocks per CU: 1 -> 64, 3x3, 1003520 pixels 67.8 against 75.4 us
+// on the implicit GEMM, 401408 31.0 and 31.3, 100352 12.1 and 10.6; 3 -> 48, 3x3
+// stride 2 17.6 and 12.7 at 100352 pixels, 91.5 and 85.3 at 1003520.
 // NHIP_CONV_SMALLK=0 turns it off, =2 takes it for every shape it supports
 // (tests).
 bool smallk_supported(const nhip_conv_plan* p, int n, int h, int w, int oh, int ow) {
@@ -224,7 +228,9 @@ bool smallk_supported(const nhip_conv_plan* p, int n, int h, int w, int oh, int 
   if (g.kh == 1 && g.kw == 1 && g.sh == 1 && g.sw == 1 && !g.pt && !g.pb && !g.pl && !g.pr) return false;
   const int64_t xb = (int64_t)n * g.c * h * w * 4, ob = (int64_t)n * g.k * oh * ow * 4;
   if (!(xb < (int64_t(1) << 31) && ob < (int64_t(1) << 31) && oh > 0 && ow > 0)) return false;
-  return mode == 2 || ceil_div((int64_t)n * oh * ow, 32) >= 4LL * cu_count();
+  if (mode == 2) return true;
+  const int64_t blocks = ceil_div((int64_t)n * oh * ow, 32);
+  return g.k <= 32 ? blocks >= 4LL * cu_count() : p->kred <= 16 && blocks >= 64LL * cu_count();
 }
 
 int launch_conv_smallk(const nhip_conv_plan* p, const float* in, const float* residual, float* out, int n, int h,

@@ -201,6 +201,7 @@ uint64_t conv_igemm_f32_workspace(const nhip_conv_plan* p, int n, int oh, int ow
     if (pointwise_selected(p, n, oh, ow)) return 0;
     if (pw_dma_supported(p, n, oh, ow)) return conv_pw_dma_workspace(p, n, oh, ow);
   }
+  if (igemm_selected(p, n, oh, ow)) return 0;
   return conv_split_workspace(p, n, oh, ow);
 }
 
@@ -216,6 +217,7 @@ int launch_conv_igemm_f32(const nhip_conv_plan* p, const float* in,
     if (pointwise_selected(p, n, h, w)) return launch_conv_pointwise_f32(p, in, residual, out, n, h, w, s);
     if (pw_dma_supported(p, n, h, w)) return launch_conv_pw_dma(p, in, residual, out, n, h, w, ws, ws_bytes, s);
   }
+  if (igemm_selected(p, n, oh, ow)) return launch_conv_igemm(p, in, residual, out, n, h, w, oh, ow, s);
   return launch_conv_split(p, in, residual, out, n, h, w, oh, ow, ws, ws_bytes, s);
 }
 

@@ -326,6 +326,12 @@ bool ip_dma_supported(const nhip_ip_plan* p, const float* in, int m);
 uint64_t innerproduct_dma_workspace(const nhip_ip_plan* p, int m);
 int launch_innerproduct_dma(const nhip_ip_plan* p, const float* in, float* out, int m, void* ws, uint64_t ws_bytes,
                             hipStream_t s);
+// conv_igemm.hip: fp32 convolutions with a short reduction that the split kernel
+// is slower at (no workspace).
+constexpr int kIgemmMaxKred = 112;
+bool igemm_selected(const nhip_conv_plan* p, int n, int oh, int ow);
+int launch_conv_igemm(const nhip_conv_plan* p, const float* in, const float* residual, float* out, int n, int h, int w,
+                      int oh, int ow, hipStream_t s);
 // conv_smallk.hip: fp32 convolutions with a reduction of at most 32 and at
 // most 32 output channels (network stems), one MFMA block per 32 pixels.
 bool smallk_supported(const nhip_conv_plan* p, int n, int h, int w, int oh, int ow);

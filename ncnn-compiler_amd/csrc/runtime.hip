@@ -567,15 +567,15 @@ int nhip_conv2d_f32_create(const nhip_conv_desc* d, const float* weight, const f
     const int khw = d->kernel_h * d->kernel_w;
     p->kred = C * khw;
     p->kred_pad = (int)round_up(p->kred, 16);
-    // row-major weights: the 1x1 kernels and the short-reduction one
-    const bool smallk = p->kred <= 32 && K <= 64, rows = khw == 1 || smallk;
-    if (rows) {
+    // row-major weights: the 1x1 kernels and those of short reductions
+    const bool shortk = p->kred <= kIgemmMaxKred;
+    if (khw == 1 || shortk) {
       std::vector<float> wp((size_t)p->m_pad * p->kred_pad, 0.f);
       for (int k = 0; k < K; ++k)
         std::copy(weight + (size_t)k * p->kred, weight + (size_t)(k + 1) * p->kred, wp.begin() + (size_t)k * p->kred_pad);
       st = upload(&p->weight, wp, "hipMalloc(conv weight)");
     }
-    if (st == NHIP_STATUS_SUCCESS && smallk) {  // the short-reduction kernel's taps
+    if (st == NHIP_STATUS_SUCCESS && shortk) {  // the short-reduction kernels' taps
       std::vector<int32_t> kt((size_t)p->kred_pad, 0x7fff << 16);
       for (int k = 0; k < p->kred; ++k) {
         const int c = k / khw, r = k % khw, kh = r / d->kernel_w, kw = r % d->kernel_w;
