@@ -182,9 +182,11 @@ __global__ void ip_splitk_reduce(const float* part, const float* bias,
 // A 1x1 stride-1 layer that runs faster on the split kernel than on the
 // streaming 1x1 kernel, both measured: from 176 input channels on (288 -> 80,
 // 15488 pixels: 17.9 -> 15.8 us; 448 -> 368, 6498: 37.3 -> 26.9; 168 -> 48,
-// 4356: 6.0 against 6.6), and from 48 where the planes are no multiple of four
+// 4356: 6.0 against 6.6), and from 49 where the planes are no multiple of four
 // pixels, which the streaming kernel reads one element at a time (80 -> 240,
-// 57x57 x 2: 15.1 -> 11.0; 24 -> 264, 22x22: no difference).  Up to 32768 pixels:
+// 57x57 x 2: 15.1 -> 11.0; 56 -> 168, 29x29 x 9: 11.3 -> 9.7), with 48 only up to one
+// 64 x 64 tile per four CUs (48 -> 64, 29x29 x 3: 5.0 -> 4.6; but 48 -> 168, 29x29 x
+// 9: 7.5 against 9.0; 24 -> 264, 22x22: no difference).  Up to 32768 pixels:
 // launches beyond stream more than the caches hold, and there the streaming
 // kernel's 16-byte loads win (192 -> 96, 50176 pixels: 25.3 against 29.6; 200
 // -> 40, 100352: 28.0 against 33.9; 256 -> 128, 25088: 25.4 -> 22.0).  A forced
@@ -193,7 +195,9 @@ static bool split_1x1_preferred(const nhip_conv_plan* p, int n, int oh, int ow) 
   for (const char* name : {"NHIP_POINTWISE", "NHIP_PW_CFG", "NHIP_PW_WGS", "NHIP_GEMM_DMA", "NHIP_CONV_KQ"})
     if (setting(name)) return false;
   const int64_t plane = (int64_t)oh * ow;
-  return n * plane < 32768 && (p->g.c >= 176 || (p->g.c >= 48 && plane % 4 != 0));
+  if (n * plane >= 32768 || p->g.c < 48) return false;
+  if (p->g.c >= 176) return true;
+  return plane % 4 != 0 && (p->g.c > 48 || 4 * ceil_div(n * plane, 64) * ceil_div(p->g.k, 64) <= cu_count());
 }
 
 uint64_t conv_igemm_f32_workspace(const nhip_conv_plan* p, int n, int oh, int ow) {
