@@ -513,20 +513,26 @@ bool pwdw_supported(const nhip_conv_plan* pw, const nhip_conv_plan* dw, int n, i
 }
 
 // Whether the fused kernel is also the faster one, for a caller that can run the
-// two layers instead (the graph executor): not where 96 input channels meet
-// planes of 128 or more pixels in so few workgroups that the phases, not the
-// launches, are the time: one or two images of 96 -> 576 at 14x14 take 15 us in
-// the fused kernel, 9 in the two layers' (MobileNetV2 on one 224x224 image 302 ->
-// 283 us over the graph, on two of 191x191 295 -> 279; from three images on, and
-// at 9x9, no gain).  NHIP_PWDW=2: always.
+// two layers instead (the graph executor): not where a wave's matrix instructions,
+// tiles times steps one after another, are 96 or more and the workgroups at most
+// one per eight CUs.  The phases of one workgroup are then the time (a step takes
+// 33 cycles, two waves share a SIMD: 96 are 2.8 us), while the two layers spread
+// over the CUs.  Fused / two layers in replayed graphs, us, all sizes from 6x6 to
+// 28x28: 96 -> 576 (24 steps) at 14x14, 7 tiles, one image 13.4 / 7.8; 9x9, 4 tiles
+// (96), 9.1 / 7.5; 8x8, 2 tiles, 6.9 / 7.6; 160 -> 960 (40 steps) at 9x9, 4 tiles, 11.5
+// / 7.9; 7x7, 2 tiles (80), 7.3 / 8.1; 64 -> 384 (16 steps) at 20x20, 7 tiles, 12.4 / 7.4;
+// 14x14, 4 tiles (64), 7.7 / 7.4; with more workgroups from 0.7 to 1.6 of the two
+// layers' time.  MobileNetV2 on one image, by the graph: 176x176 281 -> 272 us,
+// 144x144 275 -> 271, 130x200 290 -> 282, 224x224 302 -> 280.  NHIP_PWDW=2: always.
 bool pwdw_preferred(const nhip_conv_plan* pw, const nhip_conv_plan* dw, int n, int h, int w) {
   n = std::max(1, std::min(n, 65535));
   if (!pwdw_supported(pw, dw, n, h, w)) return false;
   if (setting_int("NHIP_PWDW", 1) == 2) return true;
   EdCfg c;
   if (!ed_config(pw->g.c, pw->g.k, h, w, dw->g.sh, &c)) return false;
-  const int oh = (h - 1) / dw->g.sh + 1;
-  return !(pw->g.c == 96 && h * w >= 128 && 8 * n * ceil_div(pw->g.k, c.sl) * ceil_div(oh, c.r) <= cu_count());
+  const int oh = (h - 1) / dw->g.sh + 1, steps = (int)round_up(pw->g.c, 16) / 4;
+  const int64_t workgroups = n * ceil_div(pw->g.k, c.sl) * ceil_div(oh, c.r);
+  return c.tq * steps < 96 || 8 * workgroups > cu_count();
 }
 
 int launch_pwdw_f32(const nhip_conv_plan* pw, const nhip_conv_plan* dw, const float* in, float* out, int n, int h,

@@ -14,6 +14,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+import ncnn_format  # noqa: E402
 import nhip  # noqa: E402
 import workloads  # noqa: E402
 from numerics import assert_close, max_rel_err  # noqa: E402
@@ -185,6 +186,31 @@ def test_few_images_are_supported(n):
     assert nhip.conv1x1_dw_supported(pw, dw, n, 14, 14)
     xd = dev(rng.uniform(-1, 1, (n, 96, 14, 14)).astype(np.float32))
     assert_close(host(nhip.conv1x1_dw_forward(pw, dw, xd)), host(dw.forward(pw.forward(xd))), RTOL, f"{n} images")
+
+
+@pytest.mark.parametrize("c,k,hw,n,fused", [
+    (96, 576, 14, 1, False), (96, 576, 14, 8, True),   # 168 matrix instructions a wave: 9 workgroups, 72
+    (96, 576, 9, 1, False), (96, 576, 8, 1, True),     # 96, 48
+    (160, 320, 10, 1, False), (160, 320, 7, 1, True),  # 160, 80
+    (64, 128, 20, 1, False), (64, 384, 14, 1, True),   # 112, 64
+])
+def test_graph_preference(c, k, hw, n, fused):
+    """The graph executor's choice: long chains of matrix instructions in few workgroups run as two layers."""
+    rng = np.random.default_rng(62)
+    m = ncnn_format.Model()
+    w1, b1 = workloads.he_normal(rng, (k, c, 1, 1), c), rng.standard_normal(k).astype(np.float32)
+    w2, b2 = workloads.he_normal(rng, (k, 1, 3, 3), 9), rng.standard_normal(k).astype(np.float32)
+    m.input("x", 0, 0, 0)
+    m.conv("e", "x", "e", w1, b1, stride=1, pad=0, act=1)
+    m.conv("d", "e", "d", w2, b2, stride=1, pad=1, act=1, depthwise=True)
+    graph = nhip.Graph(m.param_text(), bytes(m.payload), input_shapes=[(c, hw, hw)])
+    x = dev(rng.uniform(-1, 1, (n, c, hw, hw)).astype(np.float32))
+    nhip.timer_start("expand_dw")
+    got = graph.run(x)[0]
+    assert nhip.timer_stop()[0] == (1 if fused else 0)
+    pw = nhip.Conv2dF32(nhip.conv_desc(c, k, (1, 1), pad=(0, 0, 0, 0), act=R), w1, b1)
+    dw = nhip.DwConv2dF32(nhip.conv_desc(k, k, act=R, group=k), w2, b2)
+    assert_close(host(got), host(dw.forward(pw.forward(x))), RTOL, f"{c} -> {k} at {hw}x{hw}, {n} images")
 
 
 def test_expand_dw_random_shapes(nhip_env):
