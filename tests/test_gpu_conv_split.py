@@ -165,6 +165,44 @@ def test_chosen_algorithm_against_64_bits(n, c, h, w, k, taken):
     assert np.all(np.abs(got - exp) <= bound)
 
 
+# either side of each line of the rule that leaves the Winograd kernels (GFLOP of the direct convolution)
+AUTO_LINES = [(1, 32, 137, 140, 72, True), (1, 32, 139, 140, 72, False),      # 0.795, 0.807
+              (1, 176, 78, 79, 64, True), (1, 176, 79, 79, 64, False),        # 1.249, 1.265: 176 or more input channels
+              (1, 168, 70, 72, 64, False),                                    # 0.975, fewer
+              (1, 64, 134, 134, 48, True), (1, 64, 135, 135, 48, False),      # 0.993, 1.008: at most 48 output channels
+              (1, 64, 120, 120, 56, False)]                                   # 0.929, more
+
+
+@pytest.mark.parametrize("n,c,h,w,k,taken", AUTO_LINES)
+def test_where_the_chosen_algorithm_leaves_winograd(n, c, h, w, k, taken):
+    x, wt, b, res, plan = auto_layer(n, c, h, w, k, 4)
+    nhip.timer_start("conv_split_f32")
+    got = plan.forward(torch.from_numpy(x).cuda(), residual=torch.from_numpy(res).cuda()).cpu().double()
+    assert nhip.timer_stop()[0] == (1 if taken else 0)
+    ref = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(),
+                                     torch.from_numpy(b).double(), padding=1)
+    ref = (ref + torch.from_numpy(res).double()).clamp_min(0)
+    # normwise: the sums above, or Winograd F(4,3), whose transforms lose about four bits
+    assert ((got - ref).norm() / ref.norm()).item() < (1e-6 if taken else 6e-6)
+
+
+@pytest.mark.parametrize("c", [17, 24])
+def test_chosen_algorithm_non_finite_values(c):
+    n, h, w, k = 2, 9, 8, 40
+    x, wt, b, _, _ = auto_layer(n, c, h, w, k, 5)
+    plan = nhip.Conv2dF32(nhip.conv_desc(c, k), wt, b)
+    x.reshape(-1)[[3, 200, 555, 1100]] = [np.inf, -np.inf, np.nan, 3.4e38]
+    nhip.timer_start("conv_split_f32")
+    got = plan.forward(torch.from_numpy(x).cuda()).cpu().numpy()
+    assert nhip.timer_stop()[0] == 1
+    with np.errstate(all="ignore"):
+        exp = refcpu.conv2d_f32(refcpu.geom(n, c, h, w, k, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1)), x, wt, b)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(exp))
+    np.testing.assert_array_equal(got[np.isinf(exp)], exp[np.isinf(exp)])
+    fin = np.isfinite(exp)
+    np.testing.assert_allclose(got[fin], exp[fin], rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("c", [1, 5, 6, 7, 8, 9])
 def test_fewer_channels_than_an_octet(c, nhip_env):
     """One image of 6 channels: eight channel planes are more than the whole tensor."""

@@ -49,16 +49,40 @@ def _layer(case, int8_in):
     return nhip.conv_desc(c, k, ker, st, dl, pad, act=act, int8_scale_term=term), x, wt, b, scale, 60.0, 60.0 / spread
 
 
+def _fits(cfg, case):
+    """Whether the layer has the rows and columns of a split (a column segment is whole rows or sixteens)."""
+    n, c, h, w, k, ker, st, dl, pad, _, _ = case
+    oh = (h + pad[0] + pad[1] - dl[0] * (ker[0] - 1) - 1) // st[0] + 1
+    ow = (w + pad[2] + pad[3] - dl[1] * (ker[1] - 1) - 1) // st[1] + 1
+    if ker == (1, 1) and st == (1, 1):  # the image, or 1x1 planes' images, as one row
+        oh, ow = 1, (n if h * w == 1 else h * w)
+    r, cw = (int(v) for v in cfg.split(",")[:2])
+    return r <= oh and cw <= ow and (cw == ow or cw % 16 == 0)
+
+
+def _timed(layer):
+    nhip.timer_start("conv_int8_win")
+    got = run(*layer)
+    return got, nhip.timer_stop()[0]
+
+
 @pytest.mark.parametrize("int8_in", [True, False], ids=["i8", "f32"])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:5])) + f"-t{c[9]}")
 def test_window_kernel_bit_exact(case, int8_in, nhip_env):
     layer = _layer(case, int8_in)
     exp = oracle(*layer)
-    for cfg in CFGS:  # a split that does not fit the layer is ignored
+    window = case is not CASES[-1]
+    for cfg in CFGS:
+        if cfg and not _fits(cfg, case):
+            continue
         nhip_env.setenv("NHIP_INT8_WIN_CFG", cfg)
-        np.testing.assert_array_equal(run(*layer), exp, err_msg=f"split {cfg or 'chosen'}")
+        got, launches = _timed(layer)
+        np.testing.assert_array_equal(got, exp, err_msg=f"split {cfg or 'chosen'}")
+        assert launches == (1 if window else 0)
     nhip_env.setenv("NHIP_INT8_FOOTPRINT", "0")
-    np.testing.assert_array_equal(run(*layer), exp, err_msg="gather kernel")
+    got, launches = _timed(layer)
+    np.testing.assert_array_equal(got, exp, err_msg="gather kernel")
+    assert launches == 0
 
 
 @pytest.mark.parametrize("int8_in", [True, False], ids=["i8", "f32"])
