@@ -31,6 +31,7 @@ CASES = [
     (1, 20, 9, 9, 32, (1, 3), (3, 1), (1, 1), (2, 2, 1, 1), 1, 0),       # one-row kernel, padded rows
     (1, 16, 12, 40, 24, (5, 5), (2, 2), (2, 2), (4, 4, 4, 4), 101, 1),   # dilated, padding wider than a group
     (1, 600, 14, 12, 32, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 101, 0),  # deep: few pixels per window
+    (2, 109, 20, 19, 40, (5, 5), (2, 2), (1, 1), (2, 2, 2, 2), 101, 1),  # seven chunks of channels per pixel, unpadded
     (1, 1500, 9, 30, 32, (5, 5), (2, 2), (1, 1), (2, 2, 2, 2), 1, 0),    # no window fits: the gather kernel
 ]
 CFGS = ["", "1,32,1,1", "1,32,1,8", "2,16,2,2", "1,16,4,1", "3,32,1,4"]
