@@ -511,6 +511,20 @@ WinCfg win_config(const nhip_conv_plan* p, int in_is_i8, int n, int h, int w, in
   if (c.vecs)  // (any width: no runs along a row)
     for (int cw : {16, 8, 4})
       if (cw < c.ow) consider(1, cw);
+  // Not where only sixteen columns fit and a CU gets many such workgroups: each
+  // fills a window for half a matrix operand, and the gather kernel's 128 pixels,
+  // with the pass that quantizes the image, take less.  load: workgroups and a
+  // quarter of their channel blocks, per CU.  Window / gather: fp32 input, which is
+  // quantized once per window, below 5 0.7 to 1.1, above 5.25 0.99 to 2.3 (29 x 635 -> 14,
+  // 3x3 at 64x64: 396 / 183 us); int8 with two or more blocks per workgroup, below 10
+  // 0.8 to 1.0, above 11 1.26 to 1.75 (29 x 629 -> 62 at 33x33: 98 / 56 us), with one 0.7 to
+  // 1.1 up to 27.  1x1 windows have no rows to fill twice (15 x 594 -> 422 stride 2: 126
+  // / 174).
+  if (R > 0 && R * CW <= 16 && CW < c.ow && g.kh * g.kw > 1 && (!in_is_i8 || mbw > 1)) {
+    const int64_t tiles = (int64_t)c.n * ceil_div(c.oh, R) * ceil_div(c.ow, CW);
+    const int64_t load4 = tiles * (4 * ceil_div(mblocks, mbw) + mblocks);
+    if (load4 >= (in_is_i8 ? 40LL : 21LL) * cus) R = 0;
+  }
   if (R == 0) return c;
   if (const char* env = setting("NHIP_INT8_WIN_CFG")) {  // tuning: rows, columns, channel blocks, parts
     int r = 0, w4 = 0, m = 0, k = 0;

@@ -86,6 +86,17 @@ def test_window_kernel_bit_exact(case, int8_in, nhip_env):
     assert launches == 0
 
 
+@pytest.mark.parametrize("n,k,int8_in,window", [(13, 1, False, True), (14, 1, False, False), (21, 33, True, True),
+                                               (22, 33, True, False), (53, 1, True, True)])
+def test_sixteen_columns_leave_to_the_gather_kernel(n, k, int8_in, window):
+    """640 channels leave room for 16 columns, 80 tiles an image: either side of the workgroups from which the gather
+    kernel takes the layer; int8 with one channel block never leaves."""
+    layer = _layer((n, 640, 16, 80, k, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), 101, 1), int8_in)
+    got, launches = _timed(layer)
+    assert launches == (1 if window else 0)
+    np.testing.assert_array_equal(got, oracle(*layer))
+
+
 @pytest.mark.parametrize("int8_in", [True, False], ids=["i8", "f32"])
 def test_unaligned_input_and_output(int8_in):
     """Tensors at odd element offsets: the kernel's wide loads and stores take any element alignment."""
