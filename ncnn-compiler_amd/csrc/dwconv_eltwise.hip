@@ -660,9 +660,13 @@ unsigned grid_v4(int64_t n4) {
   return (unsigned)(blocks < cap ? (blocks > 0 ? blocks : 1) : cap);
 }
 
-// The vector kernels' launch for fewer than 2^31 elements; the element loops
-// take the rest.
-bool quant_v4_selected(int64_t count) { return count < (int64_t(1) << 31); }
+// The vector kernels' launch for 3072 elements per CU up to 2^31 elements; the
+// element loops take the rest.  Below, nothing is bound by memory, and the vector
+// kernels' longer chain (a channel found, its parameters, four groups) is the time:
+// requantize per channel, 104544 elements 2.2 us on the element loop against 4.0, 554216
+// 3.6 / 4.4, 903224 4.4 / 4.6, 1479680 6.0 / 5.0; quantize 180480 2.1 / 2.8, 714432 3.4 /
+// 3.6, 3354624 8.6 / 5.3; dequantize 291456 2.5 / 3.3, 839520 4.3 / 4.1 (in replayed graphs).
+bool quant_v4_selected(int64_t count) { return count >= 3072LL * cu_count() && count < (int64_t(1) << 31); }
 
 template <int OP>
 int launch_quant_v4(const char* name, const void* x, void* y, const float* isc, int isn, const float* osc, int osn,

@@ -12,7 +12,9 @@ from oracle import refcpu  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(1, 1, 1, 1), (3, 7, 1, 1), (2, 5, 1, 3), (2, 3, 2, 1), (3, 16, 7, 7), (2, 9, 13, 5), (1, 40, 64, 80), (5, 33, 31, 29)]
+SHAPES = [(1, 1, 1, 1), (3, 7, 1, 1), (2, 5, 1, 3), (2, 3, 2, 1), (3, 16, 7, 7), (2, 9, 13, 5), (1, 40, 64, 80), (5, 33, 31, 29),
+          # on the vector kernels (3072 elements per CU): each kind of plane, counts off four, the first count taken and the last not
+          (1, 1101, 51, 15), (3, 262145, 1, 1), (1, 400003, 1, 2), (11, 9973, 1, 9), (3, 1033, 15, 17), (1, 3072, 1, 256), (1, 786431, 1, 1)]
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
