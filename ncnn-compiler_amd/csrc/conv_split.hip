@@ -1,6 +1,7 @@
 // fp32 Convolution (reference ConvertConvolution fp32 path,
 // NCNNToTosa.cpp:1316-1529) as an implicit GEMM on the bf16 matrix
-// instructions with every fp32 operand split exactly into three bf16 pieces.
+// instructions with every fp32 operand as three bf16 pieces.  (Short reductions
+// are faster in fp32: conv_igemm.hip, conv_smallk.hip.)
 //
 // v_mfma_f32_32x32x16_bf16 does 16 times the work of v_mfma_f32_32x32x2_f32
 // in a cycle.  x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0),

@@ -266,7 +266,7 @@ bool dwpw_lds_supported(const nhip_conv_plan* dw, const nhip_conv_plan* pw, int 
 int launch_dwpw_lds_f32(const nhip_conv_plan* dw, const nhip_conv_plan* pw, const float* in,
                         const float* residual, float* out, int n, int h, int w, int oh, int ow, hipStream_t s);
 // conv_split.hip: implicit GEMM on the bf16 matrix instructions, the fp32
-// operands split exactly into three bf16 pieces (any fp32 convolution).
+// operands as three bf16 pieces each (any fp32 convolution).
 int conv_split_prepack(nhip_conv_plan* p, const float* weight);
 uint64_t conv_split_workspace(const nhip_conv_plan* p, int n, int oh, int ow);
 int launch_conv_split(const nhip_conv_plan* p, const float* in, const float* residual, float* out, int n, int h,
@@ -333,7 +333,7 @@ bool igemm_selected(const nhip_conv_plan* p, int n, int oh, int ow);
 int launch_conv_igemm(const nhip_conv_plan* p, const float* in, const float* residual, float* out, int n, int h, int w,
                       int oh, int ow, hipStream_t s);
 // conv_smallk.hip: fp32 convolutions with a reduction of at most 32 and at
-// most 32 output channels (network stems), one MFMA block per 32 pixels.
+// most 64 output channels (network stems), one MFMA block per 32 pixels.
 bool smallk_supported(const nhip_conv_plan* p, int n, int h, int w, int oh, int ow);
 // conv_kq.hip: fp32 3x3 (32 or 64 input channels) and 1x1 convolutions with
 // few output blocks, one workgroup per 32x32 block, the reduction over its
